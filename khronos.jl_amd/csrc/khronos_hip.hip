@@ -27,6 +27,7 @@
 
 #include "../../include/khronos_hip.h"
 #include "kh_kernels.hpp"
+#include "kh_half.hpp"
 
 namespace {
 
@@ -285,6 +286,7 @@ struct Ctx final : CtxBase {
     double ph_fwd[3][2] = {}, ph_rev[3][2] = {};
     T *epsi[3]{}, *mui[3]{};
     T *sigB[3]{}, *sigD[3]{};
+    T *sig_pair[2][3] = {};  // [group][axis]: (sigma, 1 / (1 + sigma)) per index (half_kernel)
     bool hassig[2][3] = {};  // [group (0: H, 1: E)][axis]: profile given (the reference's array exists)
     // material conductivity sigma_D (Ex,Ey,Ez) / sigma_B (Hx,Hy,Hz) on the
     // padded grid, 0 outside 1..N; cbox[e] = cells where some sigma of group e
@@ -432,6 +434,14 @@ struct Ctx final : CtxBase {
                 HIPCHK(hipMemcpyAsync(dv, h.data(), h.size() * sizeof(T), hipMemcpyHostToDevice, st));
                 HIPCHK(hipStreamSynchronize(st));
                 (which == 0 ? sigB : sigD)[a] = dv;
+                std::vector<T> h2(2 * h.size());
+                for (size_t i = 0; i < h.size(); ++i) {
+                    h2[2 * i] = h[i];
+                    h2[2 * i + 1] = T(1) / (T(1) + h[i]);
+                }
+                sig_pair[which][a] = (T *)dalloc(h2.size() * sizeof(T));
+                HIPCHK(hipMemcpyAsync(sig_pair[which][a], h2.data(), h2.size() * sizeof(T), hipMemcpyHostToDevice, st));
+                HIPCHK(hipStreamSynchronize(st));
             }
         }
         // per-voxel materials, reference geometry layout -> padded grid
@@ -870,6 +880,7 @@ struct Ctx final : CtxBase {
         int pblocks = 0;        // logical blocks of the PML kernel
     };
     Plan plan[2];
+    int zrun[2][3][2] = {};    // [group][axis]: first and last index of the longest run of zero sigma
     bool planned = false;
     bool nt = false;           // nontemporal access for single-use streams (inner kernels)
     bool src_in_pml = true;    // small FAST sources inside the PML launch (KH_SRC_LAUNCH=1: never)
@@ -933,6 +944,8 @@ struct Ctx final : CtxBase {
                 HIPCHK(hipMemcpyAsync(h.data(), e ? sigD[a] : sigB[a], h.size() * sizeof(T), hipMemcpyDeviceToHost, st));
                 HIPCHK(hipStreamSynchronize(st));
                 zero_run(h, g.n[a], P.lo[a], P.hi[a]);
+                zrun[e][a][0] = P.lo[a];
+                zrun[e][a][1] = P.hi[a];
                 any_empty |= P.lo[a] > P.hi[a];
             }
             // FAST mode runs the PML kernel over the whole grid (its sigma = 0
@@ -993,6 +1006,7 @@ struct Ctx final : CtxBase {
                             "per-voxel materials must be given for all three components or none");
             }
         }
+        plan_half_form();
         plan_materials();
         plan_xfold();
         planned = true;
@@ -1582,6 +1596,10 @@ struct Ctx final : CtxBase {
             const bool pervox = q.minv[0] != nullptr;
             const dim3 pgrid(q.per_xcd * kh::NXCD), pblk(kh::CBLK);
             const bool lut_on = pervox && use_lut[e];
+            if (half_ok && !cond && P.npslab == 1 && (nparts == 1 || fuse)) {
+                launch_half_kernel(e, q, fuse, lut_on ? 2 : pervox ? 1 : 0, snap, dfte_on);
+                return;
+            }
             // template flags: per-voxel material, conductivity C stage,
             // material bytes + table, both parts of a complex field
             void (*kfn)(kh::PmlArgs<T>);
@@ -1624,6 +1642,65 @@ struct Ctx final : CtxBase {
             }
             launch(2 * e + 1, kfn, pgrid, pblk, 0, q);
         }
+    }
+
+    // The whole-grid update of a half step as half_kernel (kh_half.hpp), with
+    // the arguments the pml_* kernels would take, while the state's arrays (E,
+    // H and the stages, 18 per part) are at most 440 MB together.  A step
+    // touches the fields and the shells' stages, about half of them, so up to
+    // there the 256 MB last-level cache carries the state from one half step
+    // to the next; past it that kernel's plain accesses only evict each other,
+    // and the pml_* kernels' nontemporal streams in round-robin order are
+    // faster.  us per step, half_kernel / pml_*, float cubes with 10-cell PML:
+    // 96 22.3 / 27.0, 128 44.0 / 49.1, 160 76.3 / 77.5, 176 (393 MB) 98.1 /
+    // 100.7, 192 (510 MB) 132 / 118, 208 182 / 155; double: 96 35.6 / 42.9, 128
+    // 70.7 / 82.5, 144 (430 MB) 95.3 / 102.6, 160 (590 MB) 144 / 131; complex
+    // float 128 x 128 x 192 with poles (453 MB) 147.5 / 142.3.
+    // KH_PML_KERNELS=1 keeps the pml_* kernels, 2 drops the line (below 4 GiB
+    // an array: the kernel's offsets are 32 bits).
+    bool half_ok = false;
+
+    void plan_half_form() {
+        const int form = env_int("KH_PML_KERNELS", 0);
+        const double array = (double)g.total * sizeof(T);
+        half_ok = mode == KH_MODE_FAST && form != 1 && array < 4294967296.0 && (form == 2 || 18.0 * nparts * array <= 440e6);
+    }
+
+    template <bool ELEC, int EPS>
+    static auto half_fn(bool two, bool pre, bool snap, bool dfte) -> void (*)(kh::HalfArgs<T>) {
+        if (two) return kh::half_kernel<T, ELEC, EPS, 2>;
+        if constexpr (ELEC) {
+            if (dfte) return pre ? kh::half_kernel<T, true, EPS, 1, true, false, true>
+                                 : kh::half_kernel<T, true, EPS, 1, false, false, true>;
+            if (snap) return pre ? kh::half_kernel<T, true, EPS, 1, true, true>
+                                 : kh::half_kernel<T, true, EPS, 1, false, true>;
+        }
+        return pre ? kh::half_kernel<T, ELEC, EPS, 1, true> : kh::half_kernel<T, ELEC, EPS, 1, false>;
+    }
+
+    void launch_half_kernel(int e, const kh::PmlArgs<T> &q, bool two, int eps, bool snap, bool dfte) {
+        kh::HalfArgs<T> h{};
+        h.q = q;
+        h.sy = (uint32_t)g.sy();
+        h.sz = (uint32_t)g.sz();
+        h.npair = (uint32_t)(g.n[0] + 1) / 2;
+        h.ncell = h.npair * (uint32_t)g.n[1] * (uint32_t)g.n[2];
+        h.dpair = kh::div_magic(h.npair);
+        h.dy = kh::div_magic((uint32_t)g.n[1]);
+        for (int a = 0; a < 3; ++a) {
+            h.n[a] = g.n[a];
+            h.zr[a][0] = zrun[e][a][0];
+            h.zr[a][1] = zrun[e][a][1];
+            h.sigp[a] = sig_pair[e][a];
+        }
+        const bool pre = q.pre_n > 0;
+        void (*fn)(kh::HalfArgs<T>);
+        if (e) fn = eps == 2 ? half_fn<true, 2>(two, pre, snap, dfte) : eps == 1 ? half_fn<true, 1>(two, pre, snap, dfte)
+                                                                              : half_fn<true, 0>(two, pre, snap, dfte);
+        else fn = eps == 2 ? half_fn<false, 2>(two, pre, false, false)
+                : eps == 1 ? half_fn<false, 1>(two, pre, false, false) : half_fn<false, 0>(two, pre, false, false);
+        h.q.per_xcd = (q.nblock + kh::NXCD - 1) / kh::NXCD;
+        launch(2 * e + 1, fn, dim3(h.q.per_xcd * kh::NXCD), dim3(kh::CBLK), 0, h);
     }
 
     // All DFT monitors of a half step, in launches of up to MAX_DFT monitors;
@@ -3003,7 +3080,8 @@ size_t footprint(const kh_sim_desc &d) {
     // conductivity: sigma plus C per part
     for (int c = 0; c < 6; ++c) arrays += (d.sigma_mat[c] != nullptr) * (1 + (d.complex_fields ? 2 : 1));
     size_t sig = 0;
-    for (int a = 0; a < 3; ++a) sig += 2 * ((size_t)g.n[a] + 2) * es;
+    // sigma per index, and with 1 / (1 + sigma)
+    for (int a = 0; a < 3; ++a) sig += 2 * ((size_t)g.n[a] + 2) * 3 * es;
     return arrays * (size_t)g.total * es + idx_bytes + sig + 256 * 64 * sizeof(double);
 }
 

@@ -1,0 +1,140 @@
+"""The cache-resident form of the FAST half steps (kh_half.hpp) against the pml_*
+kernels (KH_PML_KERNELS=1) on the device: the same operations on the same
+values, so fields, monitors and fluxes are equal bit for bit (tolerance 0).
+
+Sizes around the kernel's edges: rows of an odd number of cells, of one wave
+(128 cells), one less and one more, rows that start inside a wave, a last
+block that is nearly empty, one-cell axes, no sigma = 0 cells at all; PML on
+some axes, on none; 2D; wrapped axes in every combination with real and
+complex fields; H and E sources of every form; odd and even numbers of steps,
+as graphs and one by one.
+"""
+import math
+
+import numpy as np
+import pytest
+
+import khronos_hip as kh
+from khronos_hip.boundaries import PML, Bloch, Periodic
+
+pytestmark = pytest.mark.gpu
+
+COMPS = [kh.Ex, kh.Ey, kh.Ez, kh.Hx, kh.Hy, kh.Hz]
+
+
+def _pulse(f=1.0):
+    return kh.GaussianPulseSource(fcen=f, fwidth=1.5)
+
+
+def _build(n, precision, bcs=None, pml=(3, 3, 3), sources="point", eps="lut", media=None, monitors=True, res=10):
+    rng = np.random.default_rng(11)
+    cell = [v / res for v in n]
+    pmls = [[p / res, p / res] for p in pml]
+    pt = [0.07 * c for c in cell]
+    if n[2] == 0:
+        pmls, pt[2] = pmls[:2], 0.0
+    U = lambda comp, c, size=(0.0, 0.0, 0.0): kh.UniformSource(  # noqa: E731
+        time_profile=_pulse(), component=comp, center=list(c), size=list(size), amplitude=1.0)
+    src = {"point": [U(kh.Ez(), pt)],
+           "plane": [U(kh.Ez(), [pt[0], 0.0, 0.0], (0.0, 0.9 * cell[1], 0.9 * cell[2])), U(kh.Hy(), pt)],
+           "two": [U(kh.Ez(), pt), U(kh.Ez(), pt), U(kh.Hx(), [-v for v in pt])],
+           "clash": [U(kh.Hy(), pt), U(kh.Hy(), pt)]}.get(sources)
+    if sources == "wave":
+        kx, ky = (bcs[a][0].k if bcs and isinstance(bcs[a][0], Bloch) else 0.0 for a in (0, 1))
+        k = 2 * math.pi
+        src = [kh.PlaneWaveSource(time_profile=_pulse(), center=[0.0, 0.0, -0.1 * cell[2]],
+                                  size=[math.inf, math.inf, 0.0], k_vector=[-kx / k, -ky / k, 0.9])]
+    geo = []
+    if eps == "lut":
+        geo = [kh.Object(kh.Box([0.0, 0.1 * cell[1], 0.0], [0.5 * cell[0], 0.3 * cell[1], 9.0]), kh.Material(ε=4.0)),
+               kh.Object(kh.Box([0.0] * 3, [99.0] * 3), kh.Material(ε=1.7))]
+    elif eps == "array":
+        for _ in range(300):
+            c = [float(rng.uniform(-0.5, 0.5)) * v for v in cell]
+            geo.append(kh.Object(kh.Box(c, [0.35, 0.35, 0.35]), kh.Material(ε=float(rng.uniform(1.2, 9.0)))))
+    if media:
+        geo.insert(0, kh.Object(kh.Sphere([0.0] * 3, 0.3 * min(v for v in cell if v)),
+                                kh.Material(ε=2.0, chi3=0.5, susceptibilities=[
+                                    kh.LorentzianSusceptibility(1.1, 0.1, 0.6)])))
+    mons = []
+    if monitors:
+        mons = [kh.DFTMonitor(component=c(), center=[0.0] * 3, size=[cell[0], cell[1], 0.0], frequencies=[0.8, 1.1],
+                              decimation=3) for c in (kh.Ez, kh.Hx)]
+        mons.append(kh.DFTMonitor(component=kh.Ez(), center=[0.0] * 3, size=[0.5, 0.0, 0.0], frequencies=[0.9]))
+    return kh.Simulation(cell_size=cell, resolution=res, sources=src, geometry=geo, monitors=mons, boundaries=pmls,
+                         boundary_conditions=bcs, precision=precision)
+
+
+def _state(sim):
+    return [sim.read_field(C()) for C in COMPS] + [sim.engine.read_dft(i) for i in range(len(sim.spec.dfts))]
+
+
+def _compare(monkeypatch, runs, **kw):
+    out = []
+    for split in ("1", "0"):
+        monkeypatch.setenv("KH_PML_KERNELS", split)
+        sim = _build(**kw)
+        got = []
+        for n in runs:
+            sim.step(n)
+            got += _state(sim)
+        out.append(got)
+        sim.engine.close()
+    assert any(np.abs(a).max() > 0 for a in out[0])
+    for a, b in zip(*out):
+        assert np.array_equal(a, b), np.abs(a - b).max()
+
+
+per, pml_ = [Periodic(), Periodic()], [PML(), PML()]
+
+
+@pytest.mark.parametrize("precision", ["f32", "f64"])
+@pytest.mark.parametrize("n", [(13, 9, 11), (128, 5, 6), (127, 7, 5), (129, 6, 4), (64, 8, 7), (1, 12, 9), (20, 1, 1),
+                               (258, 3, 8), (40, 33, 28)])
+def test_sizes(monkeypatch, n, precision):
+    _compare(monkeypatch, [1, 2, 20], n=n, precision=precision, pml=tuple(min(3, v // 3) for v in n))
+
+
+@pytest.mark.parametrize("kw", [
+    dict(pml=(0, 0, 0)), dict(pml=(4, 0, 0)), dict(pml=(0, 4, 0)), dict(pml=(0, 0, 4)), dict(pml=(7, 7, 7)),
+    dict(eps="none"), dict(eps="array"), dict(sources="plane"), dict(sources="two"), dict(sources="clash"),
+    dict(media=True), dict(monitors=False, sources="plane"), dict(n=(37, 26, 0)), dict(n=(37, 26, 0), sources="two"),
+], ids=lambda kw: "-".join(f"{k}={v}" for k, v in kw.items()).replace(" ", ""))
+@pytest.mark.parametrize("precision", ["f32", "f64"])
+def test_forms(monkeypatch, kw, precision):
+    _compare(monkeypatch, [17, 33, 1], **{**dict(n=(35, 22, 19), precision=precision), **kw})
+
+
+@pytest.mark.parametrize("bloch", [False, True])
+@pytest.mark.parametrize("axes", ["x", "y", "z", "xy", "yz", "xz", "xyz"])
+@pytest.mark.parametrize("sources", ["point", "two", "wave"])
+@pytest.mark.parametrize("n", [(20, 13, 12), (21, 12, 13), (129, 6, 9)])
+def test_wrapped_axes(monkeypatch, n, sources, axes, bloch):
+    bcs = [([Bloch(k=0.7 + a)] * 2 if bloch and "xyz"[a] in axes[:2] else per) if "xyz"[a] in axes else pml_
+           for a in range(3)]
+    _compare(monkeypatch, [16, 5, 1], n=n, precision="f32", bcs=bcs, sources=sources, media=(n[0] == 20),
+             pml=tuple(0 if "xyz"[a] in axes else 2 for a in range(3)))
+
+
+def test_written_ghosts_reset_and_single_steps(monkeypatch):
+    """Fields written from the host (ghosts included), single steps and graphs,
+    and a reset in between."""
+    out = []
+    for split in ("1", "0"):
+        monkeypatch.setenv("KH_PML_KERNELS", split)
+        sim = _build((22, 15, 14), "f32")
+        rng = np.random.default_rng(3)
+        sim.step(3)
+        for code in range(6):
+            sim.engine.write_field(code, rng.standard_normal(sim.engine.field_shape(code)))
+        got = []
+        for n in (1, 1, 1, 20, 1, 33):
+            sim.step(n)
+            got += _state(sim)
+        kh.reset_fields(sim)
+        for n in (1, 18, 1, 1):
+            sim.step(n)
+            got += _state(sim)
+        out.append(got)
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)

@@ -1491,6 +1491,7 @@ struct DftArgs {
     // would have formed it
     int perx, xunit;
     double xfwd[2], xrev[2];
+    int gate;               // the launch may hold monitors not due this step
 };
 
 // 2 pi t of a DFT sample at step ts: E monitors sample at t + dt/2, H at t;
@@ -1502,81 +1503,120 @@ __device__ __forceinline__ double dft_theta(int64_t ts, T dt, int electric) {
     return (double)(T)(6.283185307179586 * t);
 }
 
+// (re, im) of one accumulator entry in one access
+template <typename ACC>
+struct DftC {
+    typedef ACC t __attribute__((ext_vector_type(2)));
+};
+
+// Frequencies a lane of dft_kernel updates (blockIdx.y selects them).
+constexpr int DFT_FREQS = 8;
+
 // All DFT monitors of one half step in one launch; a monitor not due this
 // step (ts % decimation != 0) exits (src/Kernels/Kernels.jl:465-497).
+//
+// Bound by the accumulators (32 bytes per cell and frequency in float64): a
+// lane takes DFT_FREQS frequencies of one cell and has them all in flight
+// while the timestep and the weights are still on their way.  With one lane
+// per cell looping over all frequencies, each load behind the store before it
+// and every block forming all the weights: 64^3, 20 frequencies 8.5 us, now
+// 4.8; 128 x 128 cells, complex fields, 100 frequencies 72 us, now 41
+// (5.2 TB/s); 192 x 160, two planes, 50 frequencies were at the copy rate and
+// stay there (49 us).  gate: a launch that can hold monitors not due at this
+// step reads the timestep before their accumulators.
 template <typename T, typename ACC>
 __global__ __launch_bounds__(256) void dft_kernel(DftArgs<T> p) {
-    extern __shared__ double wsh[];
+    __shared__ double wsh[2 * DFT_FREQS];
+    using C = typename DftC<ACC>::t;
     int q = 0;
     const int b = blockIdx.x;
     while (q + 1 < p.nmon && b >= p.mon[q + 1].first) ++q;
     const DftMon<T> &m = p.mon[q];
-    const int64_t ts = *p.clk + p.koff;
-    if (m.dec > 1 && (ts % m.dec) != 0) return;
-    const double theta = dft_theta(ts, p.dt, p.electric);
-    const double dts = (double)p.dt;
-    for (int k = threadIdx.x; k < m.nf; k += blockDim.x) {
-        double sn, cs;
-        sincos(m.freqs[k] * theta, &sn, &cs);
-        wsh[2 * k] = dts * cs;
-        wsh[2 * k + 1] = dts * sn;
-    }
-    __syncthreads();
+    const int k0 = blockIdx.y * DFT_FREQS, nk = min(DFT_FREQS, m.nf - k0);
+    if (nk <= 0) return;
+    if (p.gate && m.dec > 1 && (*p.clk + p.koff) % m.dec != 0) return;
     const int d0 = m.d[0], d1 = m.d[1], d2 = m.d[2];
     const int64_t ncell = (int64_t)d0 * d1 * d2;
     const int64_t cell = (int64_t)(b - m.first) * blockDim.x + threadIdx.x;
-    if (cell >= ncell) return;
-    int ix = (int)(cell % d0);
-    int64_t r = cell / d0;
-    int iy = (int)(r % d1);
-    int iz = (int)(r / d1);
-    const int gx = m.s[0] + ix, gy = m.s[1] + iy, gz = m.s[2] + iz;
-    // past grid index N+1 the reference's array holds an always-zero ghost
-    const bool in = gx <= p.n0 + 1 && gy <= p.n1 + 1 && gz <= p.n2 + 1;
-    const size_t fi = (size_t)gx + (size_t)gy * p.sy + (size_t)gz * p.sz;
-    const T *src = m.f, *srci = m.fim;
-    T mi = T(1);
-    if (m.rebuild && in) {
-        const int go = m.own == 0 ? gx : (m.own == 1 ? gy : gz);
-        if (m.sig_own[go] != T(0)) {
-            src = m.w;
-            srci = m.wim;
-        }
-        mi = m.minv ? m.minv[fi] : m.minv_s;
-    }
-    double v = in ? (double)(m.rebuild ? src[fi] / mi : src[fi]) : 0.0;
-    double u = in && m.fim ? (double)(m.rebuild ? srci[fi] / mi : srci[fi]) : 0.0;
-    if (p.perx && !m.rebuild && (gx == 0 || gx == p.n0 + 1) && gy >= 1 && gy <= p.n1 && gz >= 1 && gz <= p.n2) {
-        const bool hi = gx == p.n0 + 1;
-        const size_t si = hi ? fi - (size_t)p.n0 : fi + (size_t)p.n0;
-        const T fr = src[si], fm = m.fim ? srci[si] : T(0);
-        if (m.fim && !p.xunit) {
-            const double *ph = hi ? p.xfwd : p.xrev;
-            const double re = (double)fr, im = (double)fm;
-            v = (double)(T)(re * ph[0] - im * ph[1]);
-            u = (double)(T)(re * ph[1] + im * ph[0]);
+    const bool live = cell < ncell;
+    C *a = (C *)m.acc + (live ? cell : 0) + (int64_t)k0 * ncell;
+    C acc[DFT_FREQS];
+#pragma unroll
+    for (int k = 0; k < DFT_FREQS; ++k)
+        if (live && k < nk) acc[k] = a[k * ncell];
+    double v = 0.0, u = 0.0;
+    if (live) {
+        int ix, iy, iz;
+        if (ncell < ((int64_t)1 << 31)) {
+            const uint32_t r = (uint32_t)cell / (uint32_t)d0;
+            ix = (int)((uint32_t)cell - r * (uint32_t)d0);
+            iz = (int)(r / (uint32_t)d1);
+            iy = (int)(r - (uint32_t)iz * (uint32_t)d1);
         } else {
-            v = (double)fr;
-            u = (double)fm;
+            ix = (int)(cell % d0);
+            const int64_t r = cell / d0;
+            iy = (int)(r % d1);
+            iz = (int)(r / d1);
+        }
+        const int gx = m.s[0] + ix, gy = m.s[1] + iy, gz = m.s[2] + iz;
+        // past grid index N+1 the reference's array holds an always-zero ghost
+        const bool in = gx <= p.n0 + 1 && gy <= p.n1 + 1 && gz <= p.n2 + 1;
+        const size_t fi = (size_t)gx + (size_t)gy * p.sy + (size_t)gz * p.sz;
+        const T *src = m.f, *srci = m.fim;
+        T mi = T(1);
+        if (m.rebuild && in) {
+            const int go = m.own == 0 ? gx : (m.own == 1 ? gy : gz);
+            if (m.sig_own[go] != T(0)) {
+                src = m.w;
+                srci = m.wim;
+            }
+            mi = m.minv ? m.minv[fi] : m.minv_s;
+        }
+        v = in ? (double)(m.rebuild ? src[fi] / mi : src[fi]) : 0.0;
+        u = in && m.fim ? (double)(m.rebuild ? srci[fi] / mi : srci[fi]) : 0.0;
+        if (p.perx && !m.rebuild && (gx == 0 || gx == p.n0 + 1) && gy >= 1 && gy <= p.n1 && gz >= 1 && gz <= p.n2) {
+            const bool hi = gx == p.n0 + 1;
+            const size_t si = hi ? fi - (size_t)p.n0 : fi + (size_t)p.n0;
+            const T fr = src[si], fm = m.fim ? srci[si] : T(0);
+            if (m.fim && !p.xunit) {
+                const double *ph = hi ? p.xfwd : p.xrev;
+                const double re = (double)fr, im = (double)fm;
+                v = (double)(T)(re * ph[0] - im * ph[1]);
+                u = (double)(T)(re * ph[1] + im * ph[0]);
+            } else {
+                v = (double)fr;
+                u = (double)fm;
+            }
         }
     }
-    ACC *a = (ACC *)m.acc + 2 * cell;
-    if (m.fim) {
-        // complex field: (w_r + i w_i)(v + i u)
-        for (int k = 0; k < m.nf; ++k, a += 2 * ncell) {
-            const double wr = wsh[2 * k], wi = wsh[2 * k + 1];
-            double re = (double)a[0] + (wr * v - wi * u);
-            double im = (double)a[1] + (wr * u + wi * v);
-            a[0] = (ACC)re;
-            a[1] = (ACC)im;
-        }
-        return;
+    const int64_t ts = *p.clk + p.koff;
+    if ((int)threadIdx.x < nk) {
+        const double theta = dft_theta(ts, p.dt, p.electric);
+        const double dts = (double)p.dt;
+        double sn, cs;
+        sincos(m.freqs[k0 + threadIdx.x] * theta, &sn, &cs);
+        wsh[2 * threadIdx.x] = dts * cs;
+        wsh[2 * threadIdx.x + 1] = dts * sn;
     }
-    for (int k = 0; k < m.nf; ++k, a += 2 * ncell) {
-        double re = (double)a[0] + wsh[2 * k] * v;
-        double im = (double)a[1] + wsh[2 * k + 1] * v;
-        a[0] = (ACC)re;
-        a[1] = (ACC)im;
+    __syncthreads();
+    if (!live) return;
+#pragma unroll
+    for (int k = 0; k < DFT_FREQS; ++k) {
+        if (k >= nk) break;
+        const double wr = wsh[2 * k], wi = wsh[2 * k + 1];
+        double re, im;
+        if (m.fim) {
+            // complex field: (w_r + i w_i)(v + i u)
+            re = (double)acc[k][0] + (wr * v - wi * u);
+            im = (double)acc[k][1] + (wr * u + wi * v);
+        } else {
+            re = (double)acc[k][0] + wr * v;
+            im = (double)acc[k][1] + wi * v;
+        }
+        C o;
+        o[0] = (ACC)re;
+        o[1] = (ACC)im;
+        a[k * ncell] = o;
     }
 }
 
@@ -1605,35 +1645,44 @@ struct FluxMon {
     int d[3];
 };
 
-// One block per frequency: sum over the plane of
+// Sums over a share of the plane, for frequency blockIdx.x, of
 // Re(E1 conj(H2) - E2 conj(H1)) * dA after averaging the (up to) two samples
-// across the normal axis (src/Monitors/FluxMonitor.jl:104-153).
+// across the normal axis (src/Monitors/FluxMonitor.jl:104-153): blockIdx.y
+// takes every gridDim.y-th run of 256 cells, out[k * gridDim.y + y]; the host
+// adds the shares in order.  One block per frequency left most of the chip
+// idle, and its lanes took one round trip to memory after another: 128 x 128
+// cells, 100 frequencies 307 us, now 43; 192 x 160, 50 frequencies 168, now 27.
 template <typename ACC>
 __global__ __launch_bounds__(256) void flux_kernel(FluxMon e1, FluxMon e2, FluxMon h1, FluxMon h2,
                                                    int ax, int t0, int t1, int n1, int n2, double dA,
                                                    double *out) {
+    using C = typename DftC<ACC>::t;
     const int k = blockIdx.x;
     double s = 0.0;
     const FluxMon *m[4] = {&e1, &e2, &h1, &h2};
-    for (int c = threadIdx.x; c < n1 * n2; c += blockDim.x) {
+    for (int c = (int)(blockIdx.y * blockDim.x + threadIdx.x); c < n1 * n2; c += (int)(gridDim.y * blockDim.x)) {
         int i1 = c % n1, i2 = c / n1;
-        double re[4], im[4];
+        C lo[4], hi[4];
+#pragma unroll
         for (int q = 0; q < 4; ++q) {
             const FluxMon &M = *m[q];
-            const ACC *A = (const ACC *)M.acc;
             int ii[3];
             ii[ax] = 0;
             ii[t0] = i1;
             ii[t1] = i2;
             int64_t nc = (int64_t)M.d[0] * M.d[1] * M.d[2];
             int64_t lin = ii[0] + (int64_t)M.d[0] * (ii[1] + (int64_t)M.d[1] * ii[2]);
-            const ACC *p0 = A + 2 * (lin + nc * k);
-            double r = (double)p0[0], i = (double)p0[1];
-            if (M.d[ax] >= 2) {
-                int64_t step = ax == 0 ? 1 : (ax == 1 ? (int64_t)M.d[0] : (int64_t)M.d[0] * M.d[1]);
-                const ACC *p1 = p0 + 2 * step;
-                r = (r + (double)p1[0]) / 2;
-                i = (i + (double)p1[1]) / 2;
+            const C *p0 = (const C *)M.acc + (lin + nc * k);
+            int64_t step = ax == 0 ? 1 : (ax == 1 ? (int64_t)M.d[0] : (int64_t)M.d[0] * M.d[1]);
+            lo[q] = p0[0];
+            hi[q] = M.d[ax] >= 2 ? p0[step] : lo[q];
+        }
+        double re[4], im[4];
+        for (int q = 0; q < 4; ++q) {
+            double r = (double)lo[q][0], i = (double)lo[q][1];
+            if (m[q]->d[ax] >= 2) {
+                r = (r + (double)hi[q][0]) / 2;
+                i = (i + (double)hi[q][1]) / 2;
             }
             re[q] = r;
             im[q] = i;
@@ -1643,7 +1692,7 @@ __global__ __launch_bounds__(256) void flux_kernel(FluxMon e1, FluxMon e2, FluxM
         s += v * dA;
     }
     s = block_sum(s);
-    if (threadIdx.x == 0) out[k] = s;
+    if (threadIdx.x == 0) out[(size_t)k * gridDim.y + blockIdx.y] = s;
 }
 
 // Mode overlaps of a planar monitor (src/Monitors/ModeMonitor.jl:345-507):

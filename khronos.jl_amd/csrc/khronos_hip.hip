@@ -1755,6 +1755,7 @@ struct Ctx final : CtxBase {
             q.koff = koff;
             q.dt = dt;
             q.electric = electric ? 1 : 0;
+            q.gate = dft_gate_device ? 1 : 0;
             q.n0 = g.n[0]; q.n1 = g.n[1]; q.n2 = g.n[2];
             q.sy = g.sy();
             q.sz = g.sz();
@@ -1764,8 +1765,8 @@ struct Ctx final : CtxBase {
                 q.xfwd[k] = ph_fwd[0][k];
                 q.xrev[k] = ph_rev[0][k];
             }
-            const size_t shm = (size_t)nfmax * 2 * sizeof(double);
-            launch(4, acc64 ? kh::dft_kernel<T, double> : kh::dft_kernel<T, T>, dim3(blocks), dim3(256), shm, q);
+            const dim3 grid((unsigned)blocks, (unsigned)((nfmax + kh::DFT_FREQS - 1) / kh::DFT_FREQS));
+            launch(4, acc64 ? kh::dft_kernel<T, double> : kh::dft_kernel<T, T>, grid, dim3(256), 0, q);
             ++(capturing ? cap_dfts : n_dft);
         }
     }
@@ -2171,15 +2172,25 @@ struct Ctx final : CtxBase {
             n2 = std::min(n2, m.d[t1]);
         }
         require(nf <= NPART * 64, "too many frequencies");
+        // shares of the plane: about two cells a lane, within the partials
+        const int cells = std::max(1, n1 * n2);
+        const int shares = std::max(1, std::min(std::min((cells + 511) / 512, 64), NPART * 64 / nf));
+        const dim3 grid((unsigned)nf, (unsigned)shares);
         if (acc64)
-            hipLaunchKernelGGL(kh::flux_kernel<double>, dim3(nf), dim3(256), 0, st, fm[0], fm[1], fm[2], fm[3],
+            hipLaunchKernelGGL(kh::flux_kernel<double>, grid, dim3(256), 0, st, fm[0], fm[1], fm[2], fm[3],
                                ax, t0, t1, n1, n2, dA, partials);
         else
-            hipLaunchKernelGGL(kh::flux_kernel<T>, dim3(nf), dim3(256), 0, st, fm[0], fm[1], fm[2], fm[3],
+            hipLaunchKernelGGL(kh::flux_kernel<T>, grid, dim3(256), 0, st, fm[0], fm[1], fm[2], fm[3],
                                ax, t0, t1, n1, n2, dA, partials);
         HIPCHK(hipGetLastError());
-        HIPCHK(hipMemcpyAsync(out, partials, nf * sizeof(double), hipMemcpyDeviceToHost, st));
+        std::vector<double> part((size_t)nf * shares);
+        HIPCHK(hipMemcpyAsync(part.data(), partials, part.size() * sizeof(double), hipMemcpyDeviceToHost, st));
         HIPCHK(hipStreamSynchronize(st));
+        for (int k = 0; k < nf; ++k) {
+            double s = 0.0;
+            for (int j = 0; j < shares; ++j) s += part[(size_t)k * shares + j];
+            out[k] = s;
+        }
     }
 
     double *mode_buf = nullptr;   // mode profiles of the last overlap (grown on demand)

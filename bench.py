@@ -159,7 +159,7 @@ def dipole_bench(args):
         "roofline": {"bound": "hbm", "achieved": round(ab["E"] / (e_ms * 1e-3) / 1e9, 1) if e_ms > 0 else 0.0,
                      "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(ab["E"] / (e_ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4) if e_ms > 0 else 0.0,
-                     "traffic": None, "kernel": "pml_e_kernel<double,false,false,false>",
+                     "traffic": None, "kernel": "half_kernel<double,true> (E update)",
                      "alg_bytes_per_launch": ab["E"], "kernel_ms": round(e_ms, 5)},
     }
     eng.close()

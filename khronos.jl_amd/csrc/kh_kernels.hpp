@@ -1606,8 +1606,8 @@ struct DftC {
 // Frequencies a lane of dft_kernel updates (blockIdx.y selects them).
 constexpr int DFT_FREQS = 8;
 
-// All DFT monitors of one half step in one launch; a monitor not due this
-// step (ts % decimation != 0) exits (src/Kernels/Kernels.jl:465-497).
+// The DFT monitors due at one half step in one launch
+// (src/Kernels/Kernels.jl:465-497).
 //
 // Bound by the accumulators (32 bytes per cell and frequency in float64): a
 // lane takes DFT_FREQS frequencies of one cell and has them all in flight

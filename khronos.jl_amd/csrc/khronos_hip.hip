@@ -1703,12 +1703,13 @@ struct Ctx final : CtxBase {
         launch(2 * e + 1, fn, dim3(h.q.per_xcd * kh::NXCD), dim3(kh::CBLK), 0, h);
     }
 
-    // All DFT monitors of a half step, in launches of up to MAX_DFT monitors;
-    // each gates itself by its decimation against the device timestep.
+    // The DFT monitors due at a half step, in launches of up to MAX_DFT
+    // monitors.
     void launch_dfts(bool electric) {
         // the host knows the timestep of every launched or captured step
         // (graphs start on a multiple of every decimation): only due
-        // monitors are launched; the kernel gates itself as well
+        // monitors are launched, but for periods past the longest graph, where
+        // the kernel leaves out those not due by the device timestep (gate)
         const int64_t step_ts = ts + koff;
         std::vector<const Dft *> list;
         for (size_t i = 0; i < dfts.size(); ++i) {

@@ -1596,7 +1596,9 @@ struct Ctx final : CtxBase {
             const bool pervox = q.minv[0] != nullptr;
             const dim3 pgrid(q.per_xcd * kh::NXCD), pblk(kh::CBLK);
             const bool lut_on = pervox && use_lut[e];
-            if (half_ok && !cond && P.npslab == 1 && (nparts == 1 || fuse)) {
+            // without an inner box the one slab is the whole grid (beside an
+            // inner box a single slab is PML on one side of one axis)
+            if (half_ok && !cond && !P.inner && (nparts == 1 || fuse)) {
                 launch_half_kernel(e, q, fuse, lut_on ? 2 : pervox ? 1 : 0, snap, dfte_on);
                 return;
             }

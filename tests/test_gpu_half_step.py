@@ -29,7 +29,7 @@ def _pulse(f=1.0):
 def _build(n, precision, bcs=None, pml=(3, 3, 3), sources="point", eps="lut", media=None, monitors=True, res=10):
     rng = np.random.default_rng(11)
     cell = [v / res for v in n]
-    pmls = [[p / res, p / res] for p in pml]
+    pmls = [[v / res for v in (p if isinstance(p, tuple) else (p, p))] for p in pml]
     pt = [0.07 * c for c in cell]
     if n[2] == 0:
         pmls, pt[2] = pmls[:2], 0.0
@@ -114,6 +114,17 @@ def test_wrapped_axes(monkeypatch, n, sources, axes, bloch):
            for a in range(3)]
     _compare(monkeypatch, [16, 5, 1], n=n, precision="f32", bcs=bcs, sources=sources, media=(n[0] == 20),
              pml=tuple(0 if "xyz"[a] in axes else 2 for a in range(3)))
+
+
+@pytest.mark.parametrize("precision", ["f32", "f64"])
+@pytest.mark.parametrize("side", [(4, 0), (0, 4)], ids=["low", "high"])
+@pytest.mark.parametrize("axis", [0, 1, 2])
+def test_inner_box_with_one_slab(monkeypatch, axis, side, precision):
+    """KH_INNER=1 with PML on one side of one axis: an inner box and one slab.
+    The slab is not the whole grid, so half_kernel must leave it alone."""
+    monkeypatch.setenv("KH_INNER", "1")
+    _compare(monkeypatch, [1, 2, 20], n=(20, 12, 16), precision=precision,
+             pml=tuple(side if a == axis else 0 for a in range(3)))
 
 
 def test_written_ghosts_reset_and_single_steps(monkeypatch):

@@ -183,10 +183,12 @@ struct MatArgs {
     int64_t sy, sz;
     int npole;
     const PoleDev<T> *poles;
-    // per box cell: 1 where some pole's sigma or chi3 is non-zero, or null.
-    // Elsewhere P stays zero (it is only updated where its sigma is not), so
-    // fPD, the FAST corrections and the chi3 delta are zero and the pass would
-    // store what it read: such cells are skipped.
+    // per box cell: bit 0 where some pole's sigma or chi3 is non-zero, bit
+    // 1 + k where that of pole k < MAT_PRE is; or null.  Elsewhere P stays
+    // zero (it is only updated where its sigma is not): a pole's is not read
+    // without its bit, and without bit 0 fPD, the FAST corrections and the
+    // chi3 delta are zero too, the pass would store what it read, and the cell
+    // is skipped.
     const uint8_t *active;
     // FAST with a periodic axis: the wrapped ghost of a corrected boundary
     // cell is rewritten from the corrected linear field
@@ -1285,19 +1287,25 @@ __device__ __forceinline__ void cell_xyz(int64_t c, int64_t ncell, int d0, int d
 // but not D: where E carries D (s_o == 0) the next step's carried value is
 // short by (1 - s_p)/(1 + s_p) delta, delta = E_linear - E_stored.
 //
-// Every load of a cell (with its first MAT_PRE poles') is issued before the
-// first use of one: a small material box is bound by the trips to memory, not
-// by its bytes (a sphere in a 96^3 float64 grid, two poles: 9.7 us, now 7.1;
-// cylinders in 128 x 128 x 64 complex cells, two poles and chi3: 19.6, now
-// 14.2).
-constexpr int MAT_PRE = 2;
+// Every load of a cell (with its first PRE poles') is issued before the first
+// use of one: a small material box is bound by the trips to memory, not by its
+// bytes (a sphere in a 96^3 float64 grid, two poles: 9.7 us, now 7.1; cylinders
+// in 128 x 128 x 64 complex cells, two poles and chi3: 19.6, now 14.2).  A large
+// box is bound by its bytes: the mask says which of these poles a cell has, so
+// that none of the others' P is read (us per step of a whole run, two materials
+// with a pole each in layers, no read-ahead / all poles read / by the mask:
+// 224^3 float 427 / 435 / 394, 160^3 double 297 / 306 / 277), and PRE is no
+// more than the poles there are (128^3 double, one pole: 142.5 / 144.0 with two
+// slots, 140.9 with one).
+constexpr int MAT_PRE = 2;  // the most poles read ahead
 
-template <typename T, bool FAST, int NP>
+template <typename T, bool FAST, int NP, int PRE>
 __global__ __launch_bounds__(256) void material_kernel(MatArgs<T> p) {
     const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const int64_t ncell = (int64_t)p.n[0] * p.n[1] * p.n[2];
     if (c >= ncell) return;
-    if (p.active && !p.active[c]) return;
+    const uint32_t on = p.active ? p.active[c] : ~0u;
+    if (!on) return;
     int ux, uy, uz;
     cell_xyz(c, ncell, p.n[0], p.n[1], ux, uy, uz);
     const int g[3] = {p.lo[0] + ux, p.lo[1] + uy, p.lo[2] + uz};
@@ -1309,15 +1317,15 @@ __global__ __launch_bounds__(256) void material_kernel(MatArgs<T> p) {
 #pragma unroll
         for (int a = 0; a < 3; ++a) e[q][a] = p.E[q][a][idx];
     const T c3 = p.chi3 ? p.chi3[c] : T(0);
-    bool inb[MAT_PRE];
-    size_t kcs[MAT_PRE];
-    T ps[MAT_PRE], pp[MAT_PRE][NP][3], ppp[MAT_PRE][NP][3];
+    bool inb[PRE];
+    size_t kcs[PRE];
+    T ps[PRE], pp[PRE][NP][3], ppp[PRE][NP][3];
 #pragma unroll
-    for (int k = 0; k < MAT_PRE; ++k) {
+    for (int k = 0; k < PRE; ++k) {
         inb[k] = false;
         kcs[k] = 0;
         ps[k] = T(0);
-        if (k < p.npole) {
+        if (k < p.npole && (on & (2u << k))) {
             const PoleDev<T> &pl = p.poles[k];
             const int kx = g[0] - pl.lo[0], ky = g[1] - pl.lo[1], kz = g[2] - pl.lo[2];
             inb[k] = !(kx < 0 || ky < 0 || kz < 0 || kx >= pl.n[0] || ky >= pl.n[1] || kz >= pl.n[2]);
@@ -1435,14 +1443,14 @@ __global__ __launch_bounds__(256) void material_kernel(MatArgs<T> p) {
         for (int q = 0; q < NP; ++q)
             for (int a = 0; a < 3; ++a) sum[q][a] = T(0);
 #pragma unroll
-        for (int k = 0; k < MAT_PRE; ++k) {
+        for (int k = 0; k < PRE; ++k) {
             if (k >= p.npole) break;
             const PoleDev<T> &pl = p.poles[k];
 #pragma unroll
             for (int q = 0; q < NP; ++q)
 #pragma unroll
                 for (int a = 0; a < 3; ++a) {
-                    // outside the pole's box its P is zero: fPD += 0
+                    // where the pole is not its P is zero: fPD += 0
                     T pn = inb[k] ? pp[k][q][a] : T(0);
                     if (ps[k] != T(0)) {
                         const T pc = pn;
@@ -1453,7 +1461,7 @@ __global__ __launch_bounds__(256) void material_kernel(MatArgs<T> p) {
                     sum[q][a] = sum[q][a] + pn;
                 }
         }
-        for (int k = MAT_PRE; k < p.npole; ++k) {
+        for (int k = PRE; k < p.npole; ++k) {
             const PoleDev<T> &pl = p.poles[k];
             const int kx = g[0] - pl.lo[0], ky = g[1] - pl.lo[1], kz = g[2] - pl.lo[2];
             if (kx < 0 || ky < 0 || kz < 0 || kx >= pl.n[0] || ky >= pl.n[1] || kz >= pl.n[2]) {
@@ -1491,14 +1499,15 @@ __global__ __launch_bounds__(256) void material_mask_kernel(MatArgs<T> p, uint8_
     const int64_t r = c / p.n[0];
     const int uy = (int)(r % p.n[1]), uz = (int)(r / p.n[1]);
     const int g[3] = {p.lo[0] + ux, p.lo[1] + uy, p.lo[2] + uz};
-    bool on = p.chi3 && p.chi3[c] != T(0);
-    for (int k = 0; k < p.npole && !on; ++k) {
+    uint32_t on = p.chi3 && p.chi3[c] != T(0) ? 1 : 0;
+    for (int k = 0; k < p.npole && (k < MAT_PRE || !on); ++k) {
         const PoleDev<T> &pl = p.poles[k];
         const int kx = g[0] - pl.lo[0], ky = g[1] - pl.lo[1], kz = g[2] - pl.lo[2];
         if (kx < 0 || ky < 0 || kz < 0 || kx >= pl.n[0] || ky >= pl.n[1] || kz >= pl.n[2]) continue;
-        on = pl.sigma[(size_t)kx + (size_t)pl.n[0] * ((size_t)ky + (size_t)pl.n[1] * (size_t)kz)] != T(0);
+        if (pl.sigma[(size_t)kx + (size_t)pl.n[0] * ((size_t)ky + (size_t)pl.n[1] * (size_t)kz)] != T(0))
+            on |= k < MAT_PRE ? 1u | (2u << k) : 1u;
     }
-    active[c] = on ? 1 : 0;
+    active[c] = (uint8_t)on;
 }
 
 // Periodic / Bloch wrap of one field group along one axis

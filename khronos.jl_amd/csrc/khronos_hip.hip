@@ -823,10 +823,14 @@ struct Ctx final : CtxBase {
     void launch_material() {
         kh::MatArgs<T> q = mat_args();
         const dim3 grid((unsigned)((mcells + 255) / 256)), blk(256);
-        void (*kfn)(kh::MatArgs<T>);
-        if (nparts == 2) kfn = mode == KH_MODE_FAST ? kh::material_kernel<T, true, 2> : kh::material_kernel<T, false, 2>;
-        else kfn = mode == KH_MODE_FAST ? kh::material_kernel<T, true, 1> : kh::material_kernel<T, false, 1>;
-        launch(5, kfn, grid, blk, 0, q);
+        launch(5, q.npole > 1 ? material_fn<kh::MAT_PRE>() : material_fn<1>(), grid, blk, 0, q);
+    }
+
+    template <int PRE>
+    auto material_fn() const -> void (*)(kh::MatArgs<T>) {
+        if (nparts == 2)
+            return mode == KH_MODE_FAST ? kh::material_kernel<T, true, 2, PRE> : kh::material_kernel<T, false, 2, PRE>;
+        return mode == KH_MODE_FAST ? kh::material_kernel<T, true, 1, PRE> : kh::material_kernel<T, false, 1, PRE>;
     }
 
     kh::MatArgs<T> mat_args() const {

@@ -230,6 +230,13 @@ int kh_prepare_graphs(kh_ctx *ctx, int64_t n_steps);
  * no counterpart in the reference. */
 int kh_get_launch_counts(kh_ctx *ctx, int64_t counts[4]);
 
+/* Which of the two forms of the FAST updates the context launched or captured
+ * last: bit 0 (H) and bit 1 (E) are set where it was the form for states that
+ * the last-level cache holds, clear for any other kernel or before the first
+ * step.  Both give the same bits.  For measurement and tests; no counterpart
+ * in the reference. */
+int kh_get_update_form(kh_ctx *ctx, int32_t *form);
+
 /* Whether all queued work of the context has finished (*idle = 1), without
  * waiting; a scheduler serving many contexts polls this to keep each one's
  * stream fed.  Replaces: the task fetch of run_batch_concurrent

@@ -229,6 +229,7 @@ struct CtxBase {
     virtual void set_graph(int steps) = 0;
     virtual void prepare_graphs(int64_t n) = 0;
     virtual void launch_counts(int64_t *out) = 0;
+    virtual int32_t update_form() const = 0;
     virtual int graph_block() = 0;
     virtual void sync() = 0;
     virtual bool idle() = 0;
@@ -1010,8 +1011,8 @@ struct Ctx final : CtxBase {
                             "per-voxel materials must be given for all three components or none");
             }
         }
-        plan_half_form();
         plan_materials();
+        plan_half_form();
         plan_xfold();
         planned = true;
     }
@@ -1602,7 +1603,9 @@ struct Ctx final : CtxBase {
             const bool lut_on = pervox && use_lut[e];
             // without an inner box the one slab is the whole grid (beside an
             // inner box a single slab is PML on one side of one axis)
-            if (half_ok && !cond && !P.inner && (nparts == 1 || fuse)) {
+            const bool half = half_ok && !cond && !P.inner && (nparts == 1 || fuse);
+            half_groups = (half_groups & ~(1 << e)) | (half << e);
+            if (half) {
                 launch_half_kernel(e, q, fuse, lut_on ? 2 : pervox ? 1 : 0, snap, dfte_on);
                 return;
             }
@@ -1651,25 +1654,53 @@ struct Ctx final : CtxBase {
     }
 
     // The whole-grid update of a half step as half_kernel (kh_half.hpp), with
-    // the arguments the pml_* kernels would take, while the state's arrays (E,
-    // H and the stages, 18 per part) are at most 440 MB together.  A step
-    // touches the fields and the shells' stages, about half of them, so up to
-    // there the 256 MB last-level cache carries the state from one half step
-    // to the next; past it that kernel's plain accesses only evict each other,
-    // and the pml_* kernels' nontemporal streams in round-robin order are
-    // faster.  us per step, half_kernel / pml_*, float cubes with 10-cell PML:
-    // 96 22.3 / 27.0, 128 44.0 / 49.1, 160 76.3 / 77.5, 176 (393 MB) 98.1 /
-    // 100.7, 192 (510 MB) 132 / 118, 208 182 / 155; double: 96 35.6 / 42.9, 128
-    // 70.7 / 82.5, 144 (430 MB) 95.3 / 102.6, 160 (590 MB) 144 / 131; complex
-    // float 128 x 128 x 192 with poles (453 MB) 147.5 / 142.3.
+    // the arguments the pml_* kernels would take, while a step touches at most
+    // HALF_BYTES (step_bytes).  Up to there the 256 MB last-level cache carries
+    // most of it from one half step to the next; past it that kernel's plain
+    // accesses only evict each other, and the pml_* kernels' nontemporal
+    // streams in round-robin order are faster.  us per step, half_kernel /
+    // pml_*, 10-cell PML, MB as step_bytes counts them:
+    //   float cubes          128 (72) 38 / 48, 160 (135) 65 / 76, 176 (193) 95.4 /
+    //                        100.6, 184 (209) 118 / 117, 190 (220) 128 / 130
+    //   double cubes         120 (125) 56 / 69, 136 (174) 80 / 93, 144 (192) 85 /
+    //                        102, 148 (223) 111 / 115, 160 (257) 144 / 131
+    //   complex float, Bloch x and y: 128 x 128 x 64 (64) 45 / 48, x 136 (124)
+    //                        72 / 84, x 192 (171) 91 / 104
+    //   one pole everywhere  float 128 (166) 70 / 79, 144 (248) 116 / 107; double
+    //                        96 (142) 57 / 71, 136 (407) 180 / 175
+    //   two poles and chi3, complex: 128 x 128 x 64 (226) 115 / 108
     // KH_PML_KERNELS=1 keeps the pml_* kernels, 2 drops the line (below 4 GiB
     // an array: the kernel's offsets are 32 bits).
+    static constexpr double HALF_BYTES = 195e6;
     bool half_ok = false;
+    int32_t half_groups = 0;  // bit e: the last launch of group e's update was half_kernel
+
+    int32_t update_form() const override { return half_groups; }
+
+    // Bytes of the arrays a step reads or writes: E and H, U and W where sigma
+    // is not zero, per-voxel materials, the material pass's box; rows in whole
+    // 128-byte lines (the padding after them stays untouched).
+    double step_bytes() const {
+        const auto lines = [](double row) { return std::ceil(row / 128.0) * 128.0; };
+        const double rows = (double)g.n[1] * g.n[2], array = rows * lines((double)g.n[0] * sizeof(T));
+        double b = 6.0 * nparts * array;
+        for (int e = 0; e < 2; ++e) {
+            for (int a = 0; a < 3; ++a)
+                b += 2.0 * nparts * array * (g.n[a] - (zrun[e][a][1] - zrun[e][a][0] + 1)) / g.n[a];
+            if ((e ? epsi : mui)[0]) b += 3.0 * (use_lut[e] ? rows * lines((double)g.n[0]) : array);
+        }
+        if (mat) {
+            const int per = (fpd[0][0][0] ? 6 * nparts : 0) + (chi3_dev ? 1 : 0) + (delta[0][0] ? 3 * nparts : 0);
+            b += (double)mcells * per * sizeof(T);
+            for (auto &q : poles) b += (double)q.n[0] * q.n[1] * q.n[2] * (1 + 6 * nparts) * sizeof(T);
+        }
+        return b;
+    }
 
     void plan_half_form() {
         const int form = env_int("KH_PML_KERNELS", 0);
         const double array = (double)g.total * sizeof(T);
-        half_ok = mode == KH_MODE_FAST && form != 1 && array < 4294967296.0 && (form == 2 || 18.0 * nparts * array <= 440e6);
+        half_ok = mode == KH_MODE_FAST && form != 1 && array < 4294967296.0 && (form == 2 || step_bytes() <= HALF_BYTES);
     }
 
     template <bool ELEC, int EPS>
@@ -3444,6 +3475,14 @@ int kh_get_launch_counts(kh_ctx *ctx, int64_t counts[4]) {
         CTX_OK;
         require(counts != nullptr, "null argument");
         ctx->impl->launch_counts(counts);
+    });
+}
+
+int kh_get_update_form(kh_ctx *ctx, int32_t *form) {
+    return guarded([&] {
+        CTX_OK;
+        require(form != nullptr, "null argument");
+        *form = ctx->impl->update_form();
     });
 }
 

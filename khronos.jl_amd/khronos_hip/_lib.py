@@ -78,6 +78,7 @@ SIGNATURES = {
     "kh_set_graph": (C.c_int, [C.c_void_p, C.c_int32]),
     "kh_prepare_graphs": (C.c_int, [C.c_void_p, C.c_int64]),
     "kh_get_launch_counts": (C.c_int, [C.c_void_p, C.c_void_p]),
+    "kh_get_update_form": (C.c_int, [C.c_void_p, C.POINTER(C.c_int32)]),
     "kh_query": (C.c_int, [C.c_void_p, C.POINTER(C.c_int32)]),
     "kh_sync": (C.c_int, [C.c_void_p]),
     "kh_get_timestep": (C.c_int, [C.c_void_p, C.POINTER(C.c_int64)]),

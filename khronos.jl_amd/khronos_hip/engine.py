@@ -178,6 +178,13 @@ class HipEngine:
         return {"graph_replays": int(out[0]), "graph_steps": int(out[1]), "eager_steps": int(out[2]),
                 "dft_launches": int(out[3])}
 
+    def update_form(self) -> int:
+        """Bit 0 (H), bit 1 (E): the update last launched or captured was
+        half_kernel (states the last-level cache holds)."""
+        v = C.c_int32()
+        _lib.check(self.lib.kh_get_update_form(self.ctx, C.byref(v)))
+        return v.value
+
     def idle(self) -> bool:
         """All queued work finished (non-blocking)."""
         v = C.c_int32()

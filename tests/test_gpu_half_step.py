@@ -127,6 +127,28 @@ def test_inner_box_with_one_slab(monkeypatch, axis, side, precision):
              pml=tuple(side if a == axis else 0 for a in range(3)))
 
 
+@pytest.mark.parametrize("n,precision,pml,pole,form", [
+    ((40, 30, 20), "f32", 5, False, 3),
+    # the same 168^3 state (400 MB of arrays): thin PML, thick PML
+    ((168, 168, 168), "f32", 10, False, 3), ((168, 168, 168), "f32", 24, False, 0),
+    # 144^3: the material pass's arrays count, the padding of rows does not
+    ((144, 144, 144), "f32", 10, False, 3), ((144, 144, 144), "f32", 10, True, 0),
+    ((144, 144, 144), "f64", 10, False, 3), ((192, 192, 192), "f32", 10, False, 0),
+], ids=str)
+def test_line_between_the_forms(n, precision, pml, pole, form):
+    """half_kernel runs where a step touches at most 195 MB: fields, stages in
+    the PML and the material pass's box, without the rows' padding."""
+    cell = [v / 20 for v in n]
+    sus = [kh.LorentzianSusceptibility(1.1, 0.1, 0.6)] if pole else []
+    geo = [kh.Object(kh.Box([0.0] * 3, [0.95 * v for v in cell]), kh.Material(ε=2.0, susceptibilities=sus))]
+    src = kh.UniformSource(time_profile=_pulse(), component=kh.Ez(), center=[0.0] * 3, size=[0.0] * 3)
+    sim = kh.Simulation(cell_size=cell, resolution=20, sources=[src], geometry=geo if pole else [],
+                        boundaries=[[pml / 20] * 2] * 3, precision=precision, setup_precision="f64")
+    sim.step(1)
+    assert sim.engine.update_form() == form
+    sim.engine.close()
+
+
 def test_written_ghosts_reset_and_single_steps(monkeypatch):
     """Fields written from the host (ghosts included), single steps and graphs,
     and a reset in between."""

@@ -219,7 +219,8 @@ int kh_set_graph(kh_ctx *ctx, int32_t steps_per_graph);
 
 /* Capture now the graphs that kh_step(ctx, n_steps) would replay from the
  * current state, without running any step, so that a timed kh_step replays
- * graphs captured beforehand.  No counterpart in the reference (its graphs
+ * graphs captured beforehand (a kh_step beside other contexts' steps may take
+ * the other form of the updates, see kh_get_update_form, and captures its own).  No counterpart in the reference (its graphs
  * are captured on first use, src/Kernels/Kernels.jl:40-61). */
 int kh_prepare_graphs(kh_ctx *ctx, int64_t n_steps);
 

@@ -9,6 +9,7 @@
 #include <hip/hip_ext.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdlib>
 #include <cstdio>
@@ -208,6 +209,13 @@ hipStream_t pool_stream(int dev) {
 void pool_stream_release(int dev, hipStream_t s) {
     std::lock_guard<std::mutex> lock(dpool().mu);
     dpool().streams.insert({dev, s});
+}
+
+// Bytes the steps queued on a device touch (Ctx::step_bytes of every context
+// whose stream has not been seen idle since its last kh_step).
+std::atomic<int64_t> &in_flight(int dev) {
+    static std::atomic<int64_t> bytes[64];
+    return bytes[dev & 63];
 }
 
 struct DevBuf {
@@ -433,7 +441,7 @@ struct Ctx final : CtxBase {
                 }
                 T *dv = (T *)dalloc(h.size() * sizeof(T));
                 HIPCHK(hipMemcpyAsync(dv, h.data(), h.size() * sizeof(T), hipMemcpyHostToDevice, st));
-                HIPCHK(hipStreamSynchronize(st));
+                drain();
                 (which == 0 ? sigB : sigD)[a] = dv;
                 std::vector<T> h2(2 * h.size());
                 for (size_t i = 0; i < h.size(); ++i) {
@@ -442,7 +450,7 @@ struct Ctx final : CtxBase {
                 }
                 sig_pair[which][a] = (T *)dalloc(h2.size() * sizeof(T));
                 HIPCHK(hipMemcpyAsync(sig_pair[which][a], h2.data(), h2.size() * sizeof(T), hipMemcpyHostToDevice, st));
-                HIPCHK(hipStreamSynchronize(st));
+                drain();
             }
         }
         // per-voxel materials, reference geometry layout -> padded grid
@@ -467,7 +475,7 @@ struct Ctx final : CtxBase {
         partials = (double *)dalloc(NPART * 64 * sizeof(double));
         clk = (int64_t *)dalloc(256);
         graph_steps = env_int("KH_GRAPH_STEPS", 16);
-        HIPCHK(hipStreamSynchronize(st));
+        drain();
     }
 
     // reference geometry layout (component voxel count, no ghosts) -> the
@@ -481,7 +489,7 @@ struct Ctx final : CtxBase {
                 for (int i = 1; i <= g.n[0]; ++i)
                     h[g.lin(i, j, k)] = ps[(size_t)(i - 1) + (size_t)cnt[0] * ((size_t)(j - 1) + (size_t)cnt[1] * (k - 1))];
         HIPCHK(hipMemcpyAsync(dv, h.data(), h.size() * sizeof(T), hipMemcpyHostToDevice, st));
-        HIPCHK(hipStreamSynchronize(st));
+        drain();
     }
 
     // widen box b (lo[3], hi[3]) to the cells 1..N where ps (geometry layout)
@@ -508,11 +516,14 @@ struct Ctx final : CtxBase {
         drop_checkpoints();
         require(a != nullptr, "eps_inv array is null");
         require(epsi[comp] != nullptr, "the context has no per-voxel permittivity (create it with eps_inv arrays)");
-        HIPCHK(hipStreamSynchronize(st));
+        drain();
         upload_material(epsi[comp], comp, (const T *)a);
         const bool was = use_lut[1];
         rebuild_lut(1);
-        if (was != use_lut[1]) drop_graph();  // captured launches name the kernel variant
+        if (was != use_lut[1]) {
+            drop_graph();  // captured launches name the kernel variant
+            if (planned) plan_half_form();
+        }
     }
 
     // Table form of group e's per-voxel material (all three components):
@@ -528,7 +539,7 @@ struct Ctx final : CtxBase {
         std::vector<T> h(n);
         for (int a = 0; a < 3; ++a) {
             HIPCHK(hipMemcpyAsync(h.data(), src[a], n * sizeof(T), hipMemcpyDeviceToHost, st));
-            HIPCHK(hipStreamSynchronize(st));
+            drain();
             T last = T(0);
             int li = -1;
             for (size_t i = 0; i < n; ++i) {
@@ -554,12 +565,13 @@ struct Ctx final : CtxBase {
             if (!m) m = (uint8_t *)dalloc((size_t)g.total) + g.front;
             HIPCHK(hipMemcpyAsync(m, idx[a].data(), n, hipMemcpyHostToDevice, st));
         }
-        HIPCHK(hipStreamSynchronize(st));
+        drain();
         use_lut[e] = true;
     }
 
     ~Ctx() override {
         if (st) (void)hipStreamSynchronize(st);
+        note_idle();
         drop_graph();
         reap_graphs(true);
         for (auto &e : evs) { (void)hipEventDestroy(e.a); (void)hipEventDestroy(e.b); }
@@ -592,7 +604,7 @@ struct Ctx final : CtxBase {
         size_t n = (size_t)d[0] * d[1] * d[2];
         o.amp = (T *)dalloc(2 * n * sizeof(T));
         HIPCHK(hipMemcpyAsync(o.amp, amp, 2 * n * sizeof(T), hipMemcpyHostToDevice, st));
-        HIPCHK(hipStreamSynchronize(st));
+        drain();
         srcs.push_back(std::move(o));
         ++src_version;
         *id = (int32_t)srcs.size() - 1;
@@ -611,14 +623,14 @@ struct Ctx final : CtxBase {
         if (n > o.cap) {
             // a new table: captured step graphs hold the old pointer
             int64_t cap = std::max<int64_t>(n, 2 * o.cap);
-            HIPCHK(hipStreamSynchronize(st));
+            drain();
             o.wave = (double *)dalloc((size_t)(2 * cap) * sizeof(double));
             o.cap = cap;
             drop_graph();
         }
         if (n > 0) {
             HIPCHK(hipMemcpyAsync(o.wave, v, (size_t)(2 * n) * sizeof(double), hipMemcpyHostToDevice, st));
-            HIPCHK(hipStreamSynchronize(st));
+            drain();
         }
         o.nwave = n;
         ++src_version;
@@ -650,7 +662,7 @@ struct Ctx final : CtxBase {
         m.freqs = (double *)dalloc(nf * sizeof(double));
         HIPCHK(hipMemcpyAsync(m.freqs, f, nf * sizeof(double), hipMemcpyHostToDevice, st));
         m.acc = dalloc((size_t)m.ncell * nf * 2 * (acc64 ? sizeof(double) : sizeof(T)));
-        HIPCHK(hipStreamSynchronize(st));
+        drain();
         dfts.push_back(m);
         *id = (int32_t)dfts.size() - 1;
         if (planned) {  // after kh_reset: the DFT period may change
@@ -686,7 +698,7 @@ struct Ctx final : CtxBase {
                         a[(size_t)(lo[0] + i - 1) + (size_t)g.n[0] * ((size_t)(lo[1] + j - 1) + (size_t)g.n[1] * (lo[2] + k - 1))];
         T *dv = (T *)dalloc(h.size() * sizeof(T));
         HIPCHK(hipMemcpyAsync(dv, h.data(), h.size() * sizeof(T), hipMemcpyHostToDevice, st));
-        HIPCHK(hipStreamSynchronize(st));
+        drain();
         return dv;
     }
 
@@ -716,7 +728,7 @@ struct Ctx final : CtxBase {
                     q.P[pt][a] = (T *)dalloc(nb);
                     q.Pp[pt][a] = (T *)dalloc(nb);
                 }
-            HIPCHK(hipStreamSynchronize(st));
+            drain();
         }
         poles.push_back(q);
         *id = (int32_t)poles.size() - 1;
@@ -741,7 +753,7 @@ struct Ctx final : CtxBase {
             T *dv = which ? q.Pp[pt][comp] : q.P[pt][comp];
             if (rd) {
                 HIPCHK(hipMemcpyAsync(h.data(), dv, nbx * sizeof(T), hipMemcpyDeviceToHost, st));
-                HIPCHK(hipStreamSynchronize(st));
+                drain();
             }
             for (int k = 0; k < q.n[2]; ++k)
                 for (int j = 0; j < q.n[1]; ++j)
@@ -754,7 +766,7 @@ struct Ctx final : CtxBase {
                     }
             if (!rd) {
                 HIPCHK(hipMemcpyAsync(dv, h.data(), nbx * sizeof(T), hipMemcpyHostToDevice, st));
-                HIPCHK(hipStreamSynchronize(st));
+                drain();
             }
         }
     }
@@ -812,7 +824,7 @@ struct Ctx final : CtxBase {
         hipLaunchKernelGGL(kh::material_mask_kernel<T>, dim3((unsigned)((mcells + 255) / 256)), dim3(256), 0, st, q,
                            mat_active);
         HIPCHK(hipGetLastError());
-        HIPCHK(hipStreamSynchronize(st));
+        drain();
     }
 
     // cells of the material box the pass updates (null: all); dropped for
@@ -947,7 +959,7 @@ struct Ctx final : CtxBase {
                 // all transfers go through the context stream: it is non-blocking, so
                 // the legacy null stream would not be ordered after its memsets
                 HIPCHK(hipMemcpyAsync(h.data(), e ? sigD[a] : sigB[a], h.size() * sizeof(T), hipMemcpyDeviceToHost, st));
-                HIPCHK(hipStreamSynchronize(st));
+                drain();
                 zero_run(h, g.n[a], P.lo[a], P.hi[a]);
                 zrun[e][a][0] = P.lo[a];
                 zrun[e][a][1] = P.hi[a];
@@ -1409,7 +1421,7 @@ struct Ctx final : CtxBase {
             if ((int)l.size() != srcl_n[e]) drop_graph();  // the count is a launch argument
             srcl_n[e] = (int)l.size();
         }
-        HIPCHK(hipStreamSynchronize(st));
+        drain();
         srcl_version = src_version;
     }
 
@@ -1603,8 +1615,8 @@ struct Ctx final : CtxBase {
             const bool lut_on = pervox && use_lut[e];
             // without an inner box the one slab is the whole grid (beside an
             // inner box a single slab is PML on one side of one axis)
-            const bool half = half_ok && !cond && !P.inner && (nparts == 1 || fuse);
-            half_groups = (half_groups & ~(1 << e)) | (half << e);
+            const bool half = half_on && !cond && !P.inner && (nparts == 1 || fuse);
+            if (half_on) half_groups = (half_groups & ~(1 << e)) | (half << e);
             if (half) {
                 launch_half_kernel(e, q, fuse, lut_on ? 2 : pervox ? 1 : 0, snap, dfte_on);
                 return;
@@ -1669,25 +1681,55 @@ struct Ctx final : CtxBase {
     //   one pole everywhere  float 128 (166) 70 / 79, 144 (248) 116 / 107; double
     //                        96 (142) 57 / 71, 136 (407) 180 / 175
     //   two poles and chi3, complex: 128 x 128 x 64 (226) 115 / 108
+    // Contexts that step at the same time share the cache, so the line is for
+    // all of a device's contexts that have steps queued (in_flight), and each
+    // call that launches steps asks again (choose_form; the results do not
+    // depend on the answer).  us per step of all, half_kernel / pml_* / by the
+    // line, float: 6 x 64^3 37 / 47 / 37, 2 x 144^3 113 / 105 / 105, 3 x 160^3
+    // 263 / 201 / 205, 4 x 176^3 505 / 396 / 395.  The walk back of an adjoint
+    // sweep on its own stream counts as much as the re-run beside it.
     // KH_PML_KERNELS=1 keeps the pml_* kernels, 2 drops the line (below 4 GiB
     // an array: the kernel's offsets are 32 bits).
     static constexpr double HALF_BYTES = 195e6;
-    bool half_ok = false;
-    int32_t half_groups = 0;  // bit e: the last launch of group e's update was half_kernel
+    bool half_ok = false;           // half_kernel can run on this context
+    bool half_any = false;          // without a line
+    double half_bytes = 0.0;        // step_bytes()
+    bool half_on = false;           // chosen for the steps being launched
+    int32_t half_groups = 0;        // bit e: with half_on, group e's update is half_kernel
+    std::atomic<int64_t> queued{0};  // this context's share of in_flight(dev)
 
-    int32_t update_form() const override { return half_groups; }
+    int32_t update_form() const override { return half_on ? half_groups : 0; }
+
+    // beside: bytes that other work of this context touches at the same time
+    void choose_form(double beside = 0.0) {
+        const double others = (double)(in_flight(dev).load() - queued.load()) + beside;
+        half_on = half_ok && (half_any || half_bytes + others <= HALF_BYTES);
+    }
+
+    void note_queued() {
+        int64_t none = 0;
+        const int64_t b = (int64_t)half_bytes;
+        if (queued.compare_exchange_strong(none, b)) in_flight(dev) += b;
+    }
+
+    void note_idle() {
+        const int64_t b = queued.exchange(0);
+        if (b) in_flight(dev) -= b;
+    }
 
     // Bytes of the arrays a step reads or writes: E and H, U and W where sigma
     // is not zero, per-voxel materials, the material pass's box; rows in whole
     // 128-byte lines (the padding after them stays untouched).
     double step_bytes() const {
-        const auto lines = [](double row) { return std::ceil(row / 128.0) * 128.0; };
-        const double rows = (double)g.n[1] * g.n[2], array = rows * lines((double)g.n[0] * sizeof(T));
+        const auto of = [&](double elem) {
+            return (double)g.n[1] * g.n[2] * std::min(std::ceil(g.n[0] * elem / 128.0) * 128.0, g.px * elem);
+        };
+        const double array = of(sizeof(T));
         double b = 6.0 * nparts * array;
         for (int e = 0; e < 2; ++e) {
             for (int a = 0; a < 3; ++a)
                 b += 2.0 * nparts * array * (g.n[a] - (zrun[e][a][1] - zrun[e][a][0] + 1)) / g.n[a];
-            if ((e ? epsi : mui)[0]) b += 3.0 * (use_lut[e] ? rows * lines((double)g.n[0]) : array);
+            if ((e ? epsi : mui)[0]) b += 3.0 * (use_lut[e] ? of(1) : array);
         }
         if (mat) {
             const int per = (fpd[0][0][0] ? 6 * nparts : 0) + (chi3_dev ? 1 : 0) + (delta[0][0] ? 3 * nparts : 0);
@@ -1700,7 +1742,9 @@ struct Ctx final : CtxBase {
     void plan_half_form() {
         const int form = env_int("KH_PML_KERNELS", 0);
         const double array = (double)g.total * sizeof(T);
-        half_ok = mode == KH_MODE_FAST && form != 1 && array < 4294967296.0 && (form == 2 || step_bytes() <= HALF_BYTES);
+        half_ok = mode == KH_MODE_FAST && form != 1 && array < 4294967296.0;
+        half_any = form == 2;
+        half_bytes = step_bytes();
     }
 
     template <bool ELEC, int EPS>
@@ -1910,8 +1954,11 @@ struct Ctx final : CtxBase {
     }
     static constexpr int N_SHORT = 4;
     int graph_steps = 16;
-    StepGraph main_graph;
-    StepGraph short_graph[N_SHORT];
+    // one set per update form (half_on)
+    struct GraphSet {
+        StepGraph main, shorts[N_SHORT];
+    };
+    GraphSet graphs[2];
     uint64_t graph_clock = 0;
     bool graph_failed = false;
     // launch counts since the last kh_get_launch_counts
@@ -1920,8 +1967,10 @@ struct Ctx final : CtxBase {
     int64_t cap_dfts = 0;
 
     void drop_graph() {
-        retire_graph(main_graph);
-        for (auto &s : short_graph) retire_graph(s);
+        for (auto &G : graphs) {
+            retire_graph(G.main);
+            for (auto &s : G.shorts) retire_graph(s);
+        }
     }
 
     bool capture(StepGraph &sg, int len) {
@@ -1982,11 +2031,11 @@ struct Ctx final : CtxBase {
     StepGraph *pick_graph(int64_t left) {
         if (graph_len <= 0 || timing || graph_failed) return nullptr;
         const auto fits = [&](int len) { return ckpt_every <= 0 || ts % ckpt_every + len <= ckpt_every; };
-        if (left >= graph_len && ts % dft_period == 0 && fits(graph_len)) return &main_graph;
+        if (left >= graph_len && ts % dft_period == 0 && fits(graph_len)) return &graphs[half_on].main;
         if (graph_len > graph_steps && left >= graph_steps && fits(graph_steps)) {
             const int64_t ph = ts % dft_period;
-            StepGraph *hit = nullptr, *old = &short_graph[0];
-            for (auto &s : short_graph) {
+            StepGraph *hit = nullptr, *old = &graphs[half_on].shorts[0];
+            for (auto &s : graphs[half_on].shorts) {
                 if (s.phase == ph) hit = &s;
                 if (s.used < old->used) old = &s;
             }
@@ -1997,7 +2046,7 @@ struct Ctx final : CtxBase {
 
     // Capture (if needed) the graph for the current host state; false: eager.
     bool ready(StepGraph *sg, int64_t left) {
-        const int len = sg == &main_graph ? graph_len : graph_steps;
+        const int len = sg == &graphs[half_on].main ? graph_len : graph_steps;
         const bool src_now = active || last_active;
         if (!sg->x || sg->src != src_now || sg->len != len || sg->phase != ts % dft_period) {
             if (!capture(*sg, len)) {
@@ -2019,6 +2068,10 @@ struct Ctx final : CtxBase {
         stepped = true;
         sync_source_lists();
         plan_pre();
+        if (n > 0) {
+            choose_form();
+            note_queued();
+        }
         if (xfold && n > 0) xghost_stale = true;
         int64_t done = 0;
         while (done < n) {
@@ -2059,6 +2112,7 @@ struct Ctx final : CtxBase {
         }
         sync_source_lists();
         plan_pre();
+        choose_form();
         const int64_t ts0 = ts;
         const bool a0 = active, l0 = last_active;
         int64_t done = 0;
@@ -2103,11 +2157,19 @@ struct Ctx final : CtxBase {
         if (planned) plan_graph_len();
     }
 
-    void sync() override { HIPCHK(hipStreamSynchronize(st)); }
+    void sync() override { drain(); }
+
+    // everything queued on the context's stream has finished
+    void drain() {
+        HIPCHK(hipStreamSynchronize(st));
+        note_idle();
+    }
+
     bool idle() override {
         hipError_t e = hipStreamQuery(st);
         if (e == hipErrorNotReady) return false;
         HIPCHK(e);
+        note_idle();
         return true;
     }
     int64_t timestep() const override { return ts; }
@@ -2131,7 +2193,7 @@ struct Ctx final : CtxBase {
         T *o = (T *)host;
         for (int part = 0; part < nparts; ++part) {
             HIPCHK(hipMemcpyAsync(h.data(), field_ptr(comp, part), h.size() * sizeof(T), hipMemcpyDeviceToHost, st));
-            HIPCHK(hipStreamSynchronize(st));
+            drain();
             for (int k = 0; k < r[2]; ++k)
                 for (int j = 0; j < r[1]; ++j)
                     for (int i = 0; i < r[0]; ++i) {
@@ -2168,12 +2230,12 @@ struct Ctx final : CtxBase {
                         h[g.lin(i, j, k)] = in[nparts == 2 ? 2 * hi + part : hi];
                     }
             HIPCHK(hipMemcpyAsync(field_ptr(comp, part), h.data(), h.size() * sizeof(T), hipMemcpyHostToDevice, st));
-            HIPCHK(hipStreamSynchronize(st));
+            drain();
             // a written E is taken as the linear field: no chi3 deficit carried over
             if (comp < 3 && delta[part][comp])
                 HIPCHK(hipMemsetAsync(delta[part][comp], 0, (size_t)mcells * sizeof(T), st));
         }
-        HIPCHK(hipStreamSynchronize(st));
+        drain();
     }
 
     void read_dft(int id, double *host, size_t bytes) override {
@@ -2183,11 +2245,11 @@ struct Ctx final : CtxBase {
         require(bytes == n * sizeof(double), "dft buffer size mismatch");
         if (acc64) {
             HIPCHK(hipMemcpyAsync(host, m.acc, n * sizeof(double), hipMemcpyDeviceToHost, st));
-            HIPCHK(hipStreamSynchronize(st));
+            drain();
         } else {
             std::vector<T> h(n);
             HIPCHK(hipMemcpyAsync(h.data(), m.acc, n * sizeof(T), hipMemcpyDeviceToHost, st));
-            HIPCHK(hipStreamSynchronize(st));
+            drain();
             for (size_t i = 0; i < n; ++i) host[i] = (double)h[i];
         }
     }
@@ -2223,7 +2285,7 @@ struct Ctx final : CtxBase {
         HIPCHK(hipGetLastError());
         std::vector<double> part((size_t)nf * shares);
         HIPCHK(hipMemcpyAsync(part.data(), partials, part.size() * sizeof(double), hipMemcpyDeviceToHost, st));
-        HIPCHK(hipStreamSynchronize(st));
+        drain();
         for (int k = 0; k < nf; ++k) {
             double s = 0.0;
             for (int j = 0; j < shares; ++j) s += part[(size_t)k * shares + j];
@@ -2265,14 +2327,14 @@ struct Ctx final : CtxBase {
                                ax, t0, t1, n1, n2, nf, (const double *)mode_buf, dA, partials);
         HIPCHK(hipGetLastError());
         HIPCHK(hipMemcpyAsync(out, partials, (size_t)4 * nf * sizeof(double), hipMemcpyDeviceToHost, st));
-        HIPCHK(hipStreamSynchronize(st));
+        drain();
     }
 
     // growable device buffer owned by the context (the old one is freed)
     void *regrow(void *old, size_t &cap, size_t bytes) {
         if (bytes <= cap) return old;
         if (old) {
-            HIPCHK(hipStreamSynchronize(st));
+            drain();
             for (auto it = owned.begin(); it != owned.end(); ++it)
                 if (it->p == old) {
                     pool_release(dev, it->p, it->bytes);
@@ -2394,7 +2456,7 @@ struct Ctx final : CtxBase {
             HIPCHK(hipGetLastError());
         }
         HIPCHK(hipMemcpyAsync(out, n2f_out, out_bytes, hipMemcpyDeviceToHost, st));
-        HIPCHK(hipStreamSynchronize(st));
+        drain();
     }
 
     int32_t *n2f_bins = nullptr;
@@ -2436,7 +2498,7 @@ struct Ctx final : CtxBase {
         else go(std::integral_constant<int, 2>{});
         HIPCHK(hipGetLastError());
         HIPCHK(hipMemcpyAsync(out, n2f_spec, (size_t)n_bins * 8 * sizeof(double), hipMemcpyDeviceToHost, st));
-        HIPCHK(hipStreamSynchronize(st));
+        drain();
     }
 
     // every monitor's norm, in registration order: launches into separate
@@ -2457,7 +2519,7 @@ struct Ctx final : CtxBase {
                 HIPCHK(hipGetLastError());
             }
             HIPCHK(hipMemcpyAsync(part.data(), partials, (size_t)nq * NPART * sizeof(double), hipMemcpyDeviceToHost, st));
-            HIPCHK(hipStreamSynchronize(st));
+            drain();
             for (int k = 0; k < nq; ++k) {
                 double s = 0.0;
                 for (int b = 0; b < NPART; ++b) s += part[(size_t)k * NPART + b];
@@ -2480,7 +2542,7 @@ struct Ctx final : CtxBase {
                 hipLaunchKernelGGL(kh::sumsq_kernel<T>, dim3(NPART), dim3(256), 0, st, (const T *)m.acc, n, partials);
             HIPCHK(hipGetLastError());
             HIPCHK(hipMemcpyAsync(part.data(), partials, NPART * sizeof(double), hipMemcpyDeviceToHost, st));
-            HIPCHK(hipStreamSynchronize(st));
+            drain();
             double s = 0.0;
             for (double v : part) s += v;
             total += std::sqrt(s);
@@ -2572,7 +2634,7 @@ struct Ctx final : CtxBase {
     void set_checkpoints(int every) override {
         require(every >= 0, "checkpoint interval must be >= 0");
         require(every == 0 || ts == 0, "enable checkpoints before the first step or after kh_reset", KH_E_STATE);
-        HIPCHK(hipStreamSynchronize(st));
+        drain();
         for (auto &c : ck_host) c.valid = false;
         if (every == 0) {
             for (void *q : ckpt) HIPCHK(hipFree(q));
@@ -2737,7 +2799,7 @@ struct Ctx final : CtxBase {
             cot_len += (size_t)m.ncell * m.nf * 2;
         }
         // design boxes: inside cells 1..N
-        HIPCHK(hipStreamSynchronize(st));
+        drain();
         int glo[3][3], gn[3][3];
         size_t goff[3], gtot = 0;
         for (int a = 0; a < 3; ++a) {
@@ -2836,7 +2898,7 @@ struct Ctx final : CtxBase {
         adj_final = regrow(adj_final, adj_final_cap, state_bytes());
         copy_state(adj_final, nullptr, true);
         const CkHost fin{ts, active, last_active, true};
-        HIPCHK(hipStreamSynchronize(st));
+        drain();
 
         // re-runs skip the monitors; the forward state and monitors are put
         // back however the sweep ends
@@ -2859,6 +2921,8 @@ struct Ctx final : CtxBase {
             }
         } back{this, &saved, &fin};
         plan_pre();
+        choose_form(pipe ? half_bytes : 0.0);
+        note_queued();
 
         kh::BoxCopy<T> bc{};
         unsigned bmax = 1;
@@ -3042,11 +3106,11 @@ struct Ctx final : CtxBase {
         }
         if (pipe) HIPCHK(hipStreamSynchronize(st_adj));
         if (gtot) HIPCHK(hipMemcpyAsync(grad, adj_grad, gtot * sizeof(double), hipMemcpyDeviceToHost, st));
-        HIPCHK(hipStreamSynchronize(st));
+        drain();
     }
 
     void reset() override {
-        HIPCHK(hipStreamSynchronize(st));
+        drain();
         size_t fb = (size_t)g.total * sizeof(T);
         for (int part = 0; part < nparts; ++part)
             for (int a = 0; a < 3; ++a) {
@@ -3068,7 +3132,7 @@ struct Ctx final : CtxBase {
         }
         clear_material_state();
         HIPCHK(hipMemsetAsync(clk, 0, 256, st));
-        HIPCHK(hipStreamSynchronize(st));
+        drain();
         for (auto &c : ck_host) c.valid = false;
         ts = 0;
         active = true;
@@ -3096,7 +3160,7 @@ struct Ctx final : CtxBase {
     }
 
     void get_timing(double *out) override {
-        HIPCHK(hipStreamSynchronize(st));
+        drain();
         for (auto &e : evs) {
             float ms = 0.f;
             HIPCHK(hipEventElapsedTime(&ms, e.a, e.b));

@@ -149,6 +149,40 @@ def test_line_between_the_forms(n, precision, pml, pole, form):
     sim.engine.close()
 
 
+def test_contexts_in_flight_share_the_line(monkeypatch):
+    """Two 144^3 float states, about 102 MB a step each: one alone steps with
+    half_kernel, both at once with the pml kernels, chosen anew by every call.
+    A run that changes form between steps and graphs gives the same bits."""
+    kw = dict(n=(144, 144, 144), precision="f32", pml=(10, 10, 10), eps="none", res=20)
+    monkeypatch.setenv("KH_PML_KERNELS", "1")
+    ref = _build(**kw)
+    ref.step(83)
+    want = _state(ref)
+    assert ref.engine.update_form() == 0
+    ref.engine.close()
+    monkeypatch.delenv("KH_PML_KERNELS")
+    a, b = _build(**kw), _build(**kw)
+    forms = []
+    a.step(16)                        # alone
+    forms.append(a.engine.update_form())
+    b.step(33)                        # beside a's steps
+    forms.append(b.engine.update_form())
+    a.engine.sync()
+    b.step(17)                        # a has finished
+    forms.append(b.engine.update_form())
+    a.step(35)                        # beside b's
+    forms.append(a.engine.update_form())
+    got_b = b.read_field(kh.Ez())     # waits for b
+    a.step(32)
+    forms.append(a.engine.update_form())
+    b.engine.close()                  # a is in flight, b is gone
+    a.step(0)
+    assert forms == [3, 0, 3, 0, 3] and np.abs(got_b).max() > 0
+    for x, y in zip(want, _state(a)):
+        assert np.array_equal(x, y)
+    a.engine.close()
+
+
 def test_written_ghosts_reset_and_single_steps(monkeypatch):
     """Fields written from the host (ghosts included), single steps and graphs,
     and a reset in between."""

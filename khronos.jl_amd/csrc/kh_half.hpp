@@ -15,7 +15,8 @@
 //   * 1 / (1 + sigma) comes from a table, the quotient from div_by instead of
 //     a division's dozen instructions;
 //   * x + 1 / x - 1 across lanes by a wave shift, loaded only by end lanes;
-//   * the material table in LDS;
+//   * the material table in LDS, a copy per wave: waves of one block take
+//     different forms of the code, so nothing makes them meet;
 //   * accesses keep their lines (the pml_* kernels stream with nontemporal
 //     hints), and each XCD takes one contiguous eighth of the grid, so that
 //     what an XCD wrote in one half step is in its L2 or the last-level cache
@@ -141,6 +142,8 @@ __device__ __forceinline__ V half_value(V ao, V &u, V &w, V m, T K0, T K1, const
     return t;
 }
 
+constexpr int LUT_SIZE = 256;  // a byte indexes the table; four entries a lane of a wave
+
 template <typename T>
 struct HalfArgs {
     uint32_t sy, sz;       // element strides
@@ -160,8 +163,9 @@ struct HalfLane {
     static constexpr uint32_t S = sizeof(T);
     typedef T E2 __attribute__((ext_vector_type(2)));
     const HalfArgs<T> &p;
-    T *lut;
-    T lut_mine;
+    typedef T E4 __attribute__((ext_vector_type(4)));
+    T *lut;      // the wave's copy of the material table
+    E4 lut_mine; // its entries 4 lane .. 4 lane + 3
     uint32_t o, sy, sz;
     int x, y, z;
     bool live, v1, bx, by, bz;
@@ -275,10 +279,12 @@ struct HalfLane {
             if (PY && by) sgy = sig(1, y);
             if (PZ && bz) sgz = sig(2, z);
             if constexpr (EPS == 2) {
-                // the table is the oldest load in flight: the block's waves
-                // meet here with all the others behind it
-                lut[threadIdx.x] = lut_mine;
-                __syncthreads();
+                // the table is the oldest load in flight, all the others are
+                // behind it; only this wave's lanes read what it writes
+                *(E4 *)(lut + 4 * (threadIdx.x & 63)) = lut_mine;
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
                 for (int a = 0; a < 3; ++a) {
                     m[a].x = lut[mq[a] & 0xff];
                     m[a].y = lut[mq[a] >> 8];
@@ -361,10 +367,10 @@ __global__ __launch_bounds__(CBLK) void half_kernel(HalfArgs<T> args) {
     // needed; indexing the parameter itself makes the compiler copy all of it
     // to scratch memory in the larger variants
     const HalfArgs<T> &p = *(const HalfArgs<T> *)__builtin_amdgcn_kernarg_segment_ptr();
-    __shared__ T lut[EPS == 2 ? CBLK : 1];
+    __shared__ __attribute__((aligned(32))) T lut[EPS == 2 ? CBLK / 64 * LUT_SIZE : 1];
     HalfLane<T, ELEC, EPS, NP, PRE, SNAP, DFTE> k(p);
-    k.lut = lut;
-    if constexpr (EPS == 2) k.lut_mine = p.q.lut[threadIdx.x];
+    k.lut = lut + (EPS == 2 ? threadIdx.x / 64 * LUT_SIZE : 0);
+    if constexpr (EPS == 2) k.lut_mine = ((const typename decltype(k)::E4 *)p.q.lut)[threadIdx.x & 63];
     // physical block b runs on XCD b % 8: block j of XCD x is logical block
     // x * per_xcd + j
     const int j = (int)(blockIdx.x / NXCD), L = (int)(blockIdx.x % NXCD) * p.q.per_xcd + j;

@@ -29,24 +29,10 @@
 // take 3.6 us, two that copy its six arrays 6.0.
 #pragma once
 
+#include "kh_div.hpp"
 #include "kh_kernels.hpp"
 
 namespace kh {
-
-// c / d for c < 2^31 by a multiplication: d's magic number from div_magic().
-struct FastDiv {
-    uint32_t m, s;
-};
-
-inline FastDiv div_magic(uint32_t d) {
-    uint32_t l = 0;
-    while (l < 31 && (1u << l) < d) ++l;  // 2^l >= d
-    return FastDiv{(uint32_t)((((uint64_t)1 << (31 + l)) + d - 1) / d), l};
-}
-
-__device__ __forceinline__ uint32_t fdiv(uint32_t c, const FastDiv &f) {
-    return (uint32_t)(((uint64_t)c * f.m) >> (31 + f.s));
-}
 
 // the value of the lane before (AFTER: after); the end lane keeps its own
 template <bool AFTER>
@@ -63,40 +49,6 @@ __device__ __forceinline__ double lane_beside(double v) {
     const uint32_t a = (uint32_t)lane_beside<AFTER>((int)(uint32_t)q);
     const uint32_t b = (uint32_t)lane_beside<AFTER>((int)(uint32_t)(q >> 32));
     return __builtin_bit_cast(double, ((uint64_t)b << 32) | a);
-}
-
-__device__ __forceinline__ float fma_(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
-__device__ __forceinline__ double fma_(double a, double b, double c) { return __builtin_fma(a, b, c); }
-__device__ __forceinline__ float fixup_(float q, float b, float a) { return __builtin_amdgcn_div_fixupf(q, b, a); }
-__device__ __forceinline__ double fixup_(double q, double b, double a) { return __builtin_amdgcn_div_fixup(q, b, a); }
-
-// 0 < |a| < 2^-100 (2^-960): the residuals of div_by could underflow
-__device__ __forceinline__ bool tiny_(float a) {
-    return (__builtin_bit_cast(uint32_t, a) & 0x7fffffffu) - 1u < (27u << 23) - 1u;
-}
-__device__ __forceinline__ bool tiny_(double a) {
-    return ((uint32_t)(__builtin_bit_cast(uint64_t, a) >> 32) & 0x7fffffffu) < (63u << 20) && a != 0.0;
-}
-
-// (a0 / b0, a1 / b1) as IEEE division rounds them, r = 1 / b rounded to
-// nearest, 1 <= b: two residual corrections of a r (Markstein's division), half
-// the instructions of a general division.  A wave that holds a tiny value (the
-// front of a wave that is still building up) divides.  (A product with 1 / b
-// in double rounds right for float as well, in fewer instructions, but the
-// conversions are slow: 64^3 12.3 us a step against 11.3.)
-template <typename T>
-__device__ __forceinline__ void div_by(T a0, T a1, T b0, T b1, T r0, T r1, T &q0, T &q1) {
-    T p = a0 * r0, q = a1 * r1;
-    p = fma_(fma_(-b0, p, a0), r0, p);
-    q = fma_(fma_(-b1, q, a1), r1, q);
-    p = fma_(fma_(-b0, p, a0), r0, p);
-    q = fma_(fma_(-b1, q, a1), r1, q);
-    q0 = fixup_(p, b0, a0);  // infinities and NaN
-    q1 = fixup_(q, b1, a1);
-    if (__any(tiny_(a0) || tiny_(a1))) {
-        q0 = a0 / b0;
-        q1 = a1 / b1;
-    }
 }
 
 // sigma of a cell along one axis and 1 / (1 + sigma)

@@ -296,6 +296,7 @@ struct Ctx final : CtxBase {
     T *epsi[3]{}, *mui[3]{};
     T *sigB[3]{}, *sigD[3]{};
     T *sig_pair[2][3] = {};  // [group][axis]: (sigma, 1 / (1 + sigma)) per index (half_kernel)
+    bool sigma_ok = true;    // every sigma in the range of half_kernel's quotients (div_by)
     bool hassig[2][3] = {};  // [group (0: H, 1: E)][axis]: profile given (the reference's array exists)
     // material conductivity sigma_D (Ex,Ey,Ez) / sigma_B (Hx,Hy,Hz) on the
     // padded grid, 0 outside 1..N; cbox[e] = cells where some sigma of group e
@@ -445,6 +446,7 @@ struct Ctx final : CtxBase {
                 (which == 0 ? sigB : sigD)[a] = dv;
                 std::vector<T> h2(2 * h.size());
                 for (size_t i = 0; i < h.size(); ++i) {
+                    sigma_ok = sigma_ok && h[i] >= T(0) && h[i] <= T(kh::DIV_SIGMA_MAX);
                     h2[2 * i] = h[i];
                     h2[2 * i + 1] = T(1) / (T(1) + h[i]);
                 }
@@ -1689,7 +1691,9 @@ struct Ctx final : CtxBase {
     // 263 / 201 / 205, 4 x 176^3 505 / 396 / 395.  The walk back of an adjoint
     // sweep on its own stream counts as much as the re-run beside it.
     // KH_PML_KERNELS=1 keeps the pml_* kernels, 2 drops the line (below 4 GiB
-    // an array: the kernel's offsets are 32 bits).
+    // an array, the kernel's offsets are 32 bits, and with sigma in the range
+    // of its quotients: a PML profile's is, one given to kh_create can be
+    // anything).
     static constexpr double HALF_BYTES = 195e6;
     bool half_ok = false;           // half_kernel can run on this context
     bool half_any = false;          // without a line
@@ -1742,7 +1746,7 @@ struct Ctx final : CtxBase {
     void plan_half_form() {
         const int form = env_int("KH_PML_KERNELS", 0);
         const double array = (double)g.total * sizeof(T);
-        half_ok = mode == KH_MODE_FAST && form != 1 && array < 4294967296.0;
+        half_ok = mode == KH_MODE_FAST && form != 1 && sigma_ok && array < 4294967296.0;
         half_any = form == 2;
         half_bytes = step_bytes();
     }

@@ -183,6 +183,54 @@ def test_contexts_in_flight_share_the_line(monkeypatch):
     a.engine.close()
 
 
+@pytest.mark.parametrize("precision", ["f32", "f64"])
+@pytest.mark.parametrize("scale,form", [(1.0, 3), (-0.5, 0), (1e9, 0), (math.nan, 0)], ids=str)
+def test_sigma_outside_the_quotients_range(monkeypatch, scale, form, precision):
+    """half_kernel's quotients hold for 0 <= sigma <= 2^20; any other profile (as
+    kh_create takes it) steps with the pml kernels."""
+    import khronos_hip.boundaries as bnd
+    plain = bnd.compute_sigma
+    monkeypatch.setattr(bnd, "compute_sigma", lambda *a: plain(*a) * a[-1](scale))
+    sim = _build((20, 14, 13), precision)
+    sim.step(2)
+    assert sim.engine.update_form() == form
+    sim.engine.close()
+
+
+@pytest.mark.parametrize("precision", ["f32", "f64"])
+def test_values_the_quotients_special_case(monkeypatch, precision):
+    """Zeros of both signs, infinities, NaN, the largest and the smallest numbers
+    and values around the guard for tiny ones, written into the fields of a grid
+    that is all PML: the same values, and NaN in the same places."""
+    dt, guard = (np.float32, -100) if precision == "f32" else (np.float64, -960)
+    info = np.finfo(dt)
+    special = [0.0, -0.0, info.smallest_subnormal, info.tiny, 2.0 ** guard, np.nextafter(dt(2.0 ** guard), dt(0)),
+               1.5 * 2.0 ** guard, -(2.0 ** (guard - 1)), 2.0 ** (guard + 1), 1.0]
+    for wild in ([], [info.max, -info.max], [np.inf], [np.nan, -np.inf, info.max]):
+        out = []
+        for split in ("1", "0"):
+            monkeypatch.setenv("KH_PML_KERNELS", split)
+            sim = _build((21, 14, 13), precision, pml=(7, 7, 7), monitors=False)
+            rng = np.random.default_rng(7)
+            sim.step(1)
+            for code in range(6):
+                shape = sim.engine.field_shape(code)
+                v = rng.choice(np.array(special + [-x for x in special], dt), size=shape)
+                for k, x in enumerate(wild):
+                    v[3 + 4 * k, 5, 6] = x
+                sim.engine.write_field(code, v)
+            got = []
+            for n in (1, 1, 3):
+                sim.step(n)
+                got += _state(sim)
+            out.append(got)
+            assert sim.engine.update_form() == (3 if split == "0" else 0)
+            sim.engine.close()
+        for a, b in zip(*out):
+            assert np.array_equal(a, b, equal_nan=True)
+            assert np.array_equal(np.signbit(a[a == 0]), np.signbit(b[a == 0]))
+
+
 def test_written_ghosts_reset_and_single_steps(monkeypatch):
     """Fields written from the host (ghosts included), single steps and graphs,
     and a reset in between."""

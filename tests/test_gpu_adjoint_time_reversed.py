@@ -407,14 +407,17 @@ def _box3d_source_in_design(precision="f32"):
 
 
 @pytest.mark.parametrize("case", ["2d_x_pml_f64", "3d_f32", "3d_plane_source_f64", "3d_source_in_design_f32"])
-def test_snapshots_written_by_the_update_equal_separate_copies(case, monkeypatch):
+@pytest.mark.parametrize("pml_kernels", ["0", "1"], ids=["half_kernel", "pml_kernels"])
+def test_snapshots_written_by_the_update_equal_separate_copies(pml_kernels, case, monkeypatch):
     """FAST mode: the re-run's E update writes the design-box snapshot from
     its registers (W where the own-axis sigma is non-zero, else E), instead
     of a box_copy_kernel launch after each step (KH_SNAP_LAUNCH=1, read per
     gradient).  The same gradient bit for bit, captured and eager, with the
     design region in the x PML, in 3D with PML on every axis, with
     block-precomputed source corrections, and with a source inside the
-    design region (which keeps the separate copy)."""
+    design region (which keeps the separate copy).  half_kernel and the pml
+    kernels (KH_PML_KERNELS=1) each have the variant; both are run."""
+    monkeypatch.setenv("KH_PML_KERNELS", pml_kernels)
     make, n, every = {
         "2d_x_pml_f64": (lambda: slab2d_pml_design_problem(mode="fast"), 24, 41),
         "3d_f32": (lambda: box3d_problem(precision="f32", until=20.0), 20, 30),
@@ -435,6 +438,7 @@ def test_snapshots_written_by_the_update_equal_separate_copies(case, monkeypatch
     g_copy_eager = opt._time_reversed_gradient()
     monkeypatch.delenv("KH_SNAP_LAUNCH")
     g_fused_eager = opt._time_reversed_gradient()
+    assert eng.update_form() == (3 if pml_kernels == "0" else 0)
     assert np.any(g_fused != 0)
     for g in (g_copy, g_copy_eager, g_fused_eager):
         assert np.array_equal(g_fused, g)
@@ -515,3 +519,23 @@ def test_two_stream_sweep_equals_one_stream(case, monkeypatch):
     assert np.any(g_two != 0)
     for g in (g_two_again, g_one, g_one_eager, g_two_eager):
         assert np.array_equal(g_two, g)
+
+
+@pytest.mark.parametrize("case", ["2d_x_pml_f64", "3d_f32", "3d_plane_source_f64"])
+def test_gradient_of_both_update_forms(case, monkeypatch):
+    """Forward run, re-run with snapshots and objective DFTs in the E update, and
+    sweep: half_kernel against the pml kernels, the same gradient bit for bit."""
+    make, n, every = {
+        "2d_x_pml_f64": (lambda: slab2d_pml_design_problem(mode="fast"), 24, 41),
+        "3d_f32": (lambda: box3d_problem(precision="f32", until=20.0), 20, 30),
+        "3d_plane_source_f64": (lambda: plane3d_problem(), 20, 70),
+    }[case]
+    out = []
+    for pml_kernels, form in (("1", 0), ("0", 3)):
+        monkeypatch.setenv("KH_PML_KERNELS", pml_kernels)
+        opt = _time_reversed(make(), every)
+        f, g = opt(0.3 + 0.4 * np.random.default_rng(23).random(n))
+        assert opt._fwd_sim.engine.update_form() == form
+        out.append((np.asarray(f), g))
+    assert np.any(out[0][1] != 0)
+    assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])

@@ -6,7 +6,8 @@ accumulators, no material pass or periodic axis, no E source writing a
 monitor cell of its component) from the values it stores, with weights
 formed once per block of steps; dft_kernel runs only for the other monitors
 (KH_DFT_LAUNCH=1, read when a context plans its steps: every monitor in
-dft_kernel).  Both perform the same operations on the same values, so the
+dft_kernel).  half_kernel and the pml kernels (KH_PML_KERNELS=1) each have the
+variant; both are run.  Both perform the same operations on the same values, so the
 fields and every DFT agree bit for bit: 3D and 2D, FP32 and FP64, monitors
 with and without decimation, a fifth small E monitor (left to dft_kernel),
 an H monitor, a monitor under a source of its component, and a plane source
@@ -87,7 +88,9 @@ def _step(sim, n, separate):
                                                               ("f64", False, False, True),
                                                               ("f32", True, False, False),
                                                               ("f64", False, True, False)])
-def test_dft_in_e_update_equals_dft_launches(precision, two_d, plane, src_on_mon):
+@pytest.mark.parametrize("pml_kernels", ["0", "1"], ids=["half_kernel", "pml_kernels"])
+def test_dft_in_e_update_equals_dft_launches(monkeypatch, pml_kernels, precision, two_d, plane, src_on_mon):
+    monkeypatch.setenv("KH_PML_KERNELS", pml_kernels)
     fused = _scene(precision, two_d, plane, src_on_mon)
     sep = _scene(precision, two_d, plane, src_on_mon)
     fused.prepare()
@@ -106,6 +109,7 @@ def test_dft_in_e_update_equals_dft_launches(precision, two_d, plane, src_on_mon
         ns += sep.engine.launch_counts()["dft_launches"]
         for a, b in zip(_state(fused), _state(sep)):
             assert np.array_equal(a, b), done
+    assert fused.engine.update_form() == sep.engine.update_form() == (3 if pml_kernels == "0" else 0)
     _note(f"[dft in update] dft_kernel launches {nf} (E update on) vs {ns} (off) in {done} steps")
     assert nf < ns
     assert all(np.any(sep.engine.read_dft(i) != 0) for i in range(5))

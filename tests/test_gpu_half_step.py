@@ -1,6 +1,9 @@
 """The cache-resident form of the FAST half steps (kh_half.hpp) against the pml_*
 kernels (KH_PML_KERNELS=1) on the device: the same operations on the same
 values, so fields, monitors and fluxes are equal bit for bit (tolerance 0).
+Every comparison asserts which kernels ran (update_form): half_kernel in one run
+and not in the other, but for a field group without any sigma, which steps with
+the inner kernels in both and is compared as such.
 
 Sizes around the kernel's edges: rows of an odd number of cells, of one wave
 (128 cells), one less and one more, rows that start inside a wave, a last
@@ -69,16 +72,25 @@ def _state(sim):
     return [sim.read_field(C()) for C in COMPS] + [sim.engine.read_dft(i) for i in range(len(sim.spec.dfts))]
 
 
-def _compare(monkeypatch, runs, **kw):
+def _groups_with_sigma(sim):
+    """Bit 0 (H), bit 1 (E): some sigma the kernels read is not zero."""
+    sig = sim.spec.sigma or {}
+    return sum(1 << bit for bit, key in enumerate("BD")
+               if any(s is not None and np.any(np.asarray(s)[0:2 * n:2]) for s, n in zip(sig.get(key, ()), sim.spec.N)))
+
+
+def _compare(monkeypatch, runs, half=None, build=_build, **kw):
     out = []
     for split in ("1", "0"):
         monkeypatch.setenv("KH_PML_KERNELS", split)
-        sim = _build(**kw)
+        sim = build(**kw)
         got = []
         for n in runs:
             sim.step(n)
             got += _state(sim)
         out.append(got)
+        want = 0 if split == "1" else _groups_with_sigma(sim) if half is None else half
+        assert sim.engine.update_form() == want
         sim.engine.close()
     assert any(np.abs(a).max() > 0 for a in out[0])
     for a, b in zip(*out):
@@ -108,12 +120,35 @@ def test_forms(monkeypatch, kw, precision):
 @pytest.mark.parametrize("bloch", [False, True])
 @pytest.mark.parametrize("axes", ["x", "y", "z", "xy", "yz", "xz", "xyz"])
 @pytest.mark.parametrize("sources", ["point", "two", "wave"])
-@pytest.mark.parametrize("n", [(20, 13, 12), (21, 12, 13), (129, 6, 9)])
-def test_wrapped_axes(monkeypatch, n, sources, axes, bloch):
+@pytest.mark.parametrize("n,precision", [((20, 13, 12), "f32"), ((21, 12, 13), "f32"), ((129, 6, 9), "f32"),
+                                         ((20, 13, 12), "f64"), ((21, 12, 13), "f64")])
+def test_wrapped_axes(monkeypatch, n, precision, sources, axes, bloch):
     bcs = [([Bloch(k=0.7 + a)] * 2 if bloch and "xyz"[a] in axes[:2] else per) if "xyz"[a] in axes else pml_
            for a in range(3)]
-    _compare(monkeypatch, [16, 5, 1], n=n, precision="f32", bcs=bcs, sources=sources, media=(n[0] == 20),
+    _compare(monkeypatch, [16, 5, 1], n=n, precision=precision, bcs=bcs, sources=sources, media=(n[0] == 20),
              pml=tuple(0 if "xyz"[a] in axes else 2 for a in range(3)))
+
+
+def _conductor(group, precision, bloch):
+    """A block with material conductivity of one field group only."""
+    mat = kh.Material(ε=2.0, σD=1.3) if group == "E" else kh.Material(ε=2.0, σB=0.8)
+    src = [kh.UniformSource(time_profile=_pulse(), component=c(), center=[0.3, -0.2, 0.1], size=[0.0] * 3)
+           for c in (kh.Ez, kh.Hx)]
+    bcs = [[Bloch(k=0.7)] * 2, pml_, pml_] if bloch else None
+    mon = kh.DFTMonitor(component=kh.Ez(), center=[0.0] * 3, size=[1.0, 0.8, 0.0], frequencies=[0.8, 1.1])
+    return kh.Simulation(cell_size=[2.1, 1.4, 1.6], resolution=10, sources=src, monitors=[mon],
+                         geometry=[kh.Object(kh.Box([0.2, 0.0, 0.0], [0.8, 0.7, 0.5]), mat)],
+                         boundaries=[[0.0 if bloch else 0.3] * 2, [0.3] * 2, [0.3] * 2], boundary_conditions=bcs,
+                         precision=precision)
+
+
+@pytest.mark.parametrize("bloch", [False, True])
+@pytest.mark.parametrize("precision", ["f32", "f64"])
+@pytest.mark.parametrize("group,half", [("E", 1), ("H", 2)])
+def test_conductivity_in_one_group(monkeypatch, group, half, precision, bloch):
+    """The conductive group keeps the pml kernels and their C stage, the other
+    steps with half_kernel."""
+    _compare(monkeypatch, [17, 20, 1], half=half, build=_conductor, group=group, precision=precision, bloch=bloch)
 
 
 @pytest.mark.parametrize("precision", ["f32", "f64"])
@@ -123,7 +158,7 @@ def test_inner_box_with_one_slab(monkeypatch, axis, side, precision):
     """KH_INNER=1 with PML on one side of one axis: an inner box and one slab.
     The slab is not the whole grid, so half_kernel must leave it alone."""
     monkeypatch.setenv("KH_INNER", "1")
-    _compare(monkeypatch, [1, 2, 20], n=(20, 12, 16), precision=precision,
+    _compare(monkeypatch, [1, 2, 20], half=0, n=(20, 12, 16), precision=precision,
              pml=tuple(side if a == axis else 0 for a in range(3)))
 
 

@@ -1,10 +1,13 @@
-// kh_half.hpp -- the FAST half step (H or E) on the whole grid for a state that
-// the last-level cache holds (Ctx::plan_half_form has the line), without
-// conductivity: the update of the pml_* kernels with the same operations on
-// the same values (bit for bit).
+// kh_half.hpp -- the FAST half step (H or E) on the whole grid where the
+// last-level cache holds most of what a step touches (Ctx::choose_form has the
+// line), without conductivity: the update of the pml_* kernels with the same
+// operations on the same values (bit for bit).
 //
-// There a half step is not bound by HBM but by how long one wave takes and by
-// what the caches give back: a launch is one or two rounds of waves.  So
+// Up to about 64^3 float cells (two waves a SIMD) a launch is one round of waves
+// and its time is that of one wave: 5.4 us with 16.5 MB past the L2, 3.0 TB/s.
+// From about 80^3 double or 100^3 float cells on it is what the caches give
+// back: 131 x 117 x 101 float 12 waves a SIMD, 91 MB (H) and 97 MB (E) past the
+// L2 in 17-18 us, 5.4 TB/s, the address units half busy.  So
 //   * a pair's (x, y, z) comes from two multiplications (FastDiv), its
 //     accesses from a scalar base and one 32-bit offset;
 //   * which stages exist is decided by index (outside the longest run of zero
@@ -25,8 +28,8 @@
 // 11.3 us, 131 x 117 x 101 float 46.3 -> 41.3, 160 x 145 x 120 float with
 // per-voxel arrays 61.2 -> 54.7, 80^3 double 28.1 -> 20.4.  The launch shape
 // and the code gave 12.3 / 44.5 / 59.5 / 25.2 of that, the last item the rest.
-// What is left of 64^3 is launches: two dependent empty kernels of a graph
-// take 3.6 us, two that copy its six arrays 6.0.
+// Of 64^3's 11.3 us two dependent launches that copy its six arrays explain 6.0
+// (two empty ones 3.6).
 #pragma once
 
 #include "kh_div.hpp"

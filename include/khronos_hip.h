@@ -220,8 +220,9 @@ int kh_set_graph(kh_ctx *ctx, int32_t steps_per_graph);
 /* Capture now the graphs that kh_step(ctx, n_steps) would replay from the
  * current state, without running any step, so that a timed kh_step replays
  * graphs captured beforehand (a kh_step beside other contexts' steps may take
- * the other form of the updates, see kh_get_update_form, and captures its own).  No counterpart in the reference (its graphs
- * are captured on first use, src/Kernels/Kernels.jl:40-61). */
+ * the other form of the updates, see kh_get_update_form, and captures its
+ * own).  No counterpart in the reference (its graphs are captured on first
+ * use, src/Kernels/Kernels.jl:40-61). */
 int kh_prepare_graphs(kh_ctx *ctx, int64_t n_steps);
 
 /* What kh_step ran since the last call (then cleared): counts[0] graph
@@ -234,8 +235,11 @@ int kh_get_launch_counts(kh_ctx *ctx, int64_t counts[4]);
 /* Which of the two forms of the FAST updates the context launched or captured
  * last: bit 0 (H) and bit 1 (E) are set where it was the form for states that
  * the last-level cache holds, clear for any other kernel or before the first
- * step.  Both give the same bits.  For measurement and tests; no counterpart
- * in the reference. */
+ * step.  Both give the same bits.  kh_step, kh_prepare_graphs and
+ * kh_adjoint_gradient choose by what the device's contexts with steps queued
+ * touch together; a context counts until a call on it (kh_sync, kh_query, a
+ * read, kh_destroy) has seen its steps finished.  For measurement and tests; no
+ * counterpart in the reference. */
 int kh_get_update_form(kh_ctx *ctx, int32_t *form);
 
 /* Whether all queued work of the context has finished (*idle = 1), without

@@ -54,7 +54,7 @@ def cpu_baseline(spec, cores: int, budget_s: float = 12.0, warmup: int = 10, lab
     ``cores`` threads) on the same workload: ``warmup`` untimed steps, as
     run_benchmark does (src/Simulation.jl:492-527), then a bounded sample."""
     sys.path.insert(0, os.path.join(ROOT, "tests"))
-    from oracle_engine import OracleEngine  # the checker, used here only as the CPU baseline
+    from oracle_engine import OracleEngine  # the oracle, used here only as the CPU baseline
     _omp_threads(cores)
     eng = OracleEngine(spec)
     t0 = time.perf_counter()
@@ -457,7 +457,7 @@ def near2far_bench(args):
     }
     if not args.no_cpu_baseline:
         sys.path.insert(0, os.path.join(ROOT, "tests"))
-        import n2f_oracle as N  # the checker, used here only as the CPU baseline
+        import n2f_oracle as N  # the oracle, used here only as the CPU baseline
         mons = md.tangential_E_monitors + md.tangential_H_monitors
         planes = [sim.read_dft(x.monitor_data)[..., :1] for x in mons]
         sub = obs[::2]
@@ -523,7 +523,7 @@ def adjoint_line(steps: int, warmup: int, cpu: bool = True) -> dict:
     }
     if cpu:
         sys.path.insert(0, os.path.join(ROOT, "tests"))
-        from oracle_engine import OracleEngine  # the checker, used here only as the CPU baseline
+        from oracle_engine import OracleEngine  # the oracle, used here only as the CPU baseline
         cores = min(len(os.sched_getaffinity(0)), int(os.environ.get("OMP_NUM_THREADS", "16") or 16), 16)
         _omp_threads(cores)
         ref, _ = W.adjoint_bend(precision="f32", setup_precision="f64", method="frequency", engine=OracleEngine)

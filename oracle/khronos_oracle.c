@@ -1,7 +1,7 @@
 /*
  * khronos_oracle.c -- CPU restatement of the reference's time step.
  *
- * TEST INFRASTRUCTURE ONLY.  This file is the checker for the HIP library:
+ * TEST INFRASTRUCTURE ONLY.  This file is the oracle for the HIP library:
  * only tests/, __graft_entry__.smoke() and bench.py's cpu_baseline leg load it,
  * and never as the thing measured or shipped.
  *

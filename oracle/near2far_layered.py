@@ -1,6 +1,6 @@
 """Layered-medium near-to-far projection, restated in numpy.
 
-TEST INFRASTRUCTURE ONLY: the checker for khronos_hip's layered projection
+TEST INFRASTRUCTURE ONLY: the oracle for khronos_hip's layered projection
 (device spectral sums + host transfer matrices).  Only tests/ load it.
 
 It restates, step by step:

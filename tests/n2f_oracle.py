@@ -1,7 +1,7 @@
 """ctypes wrappers of the oracle's near-to-far functions (oracle/khronos_oracle.c:
 orc_green3d = green3d!, orc_near2far = the surface sum) for the tests.
 
-The oracle is the checker: tests compare the HIP library's kh_near2far with
+Tests compare the HIP library's kh_near2far with
 it, and pin it against closed forms (Maxwell's curl equations, the surface
 equivalence theorem, far-field decay).
 """
